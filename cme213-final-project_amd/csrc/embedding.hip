@@ -123,12 +123,14 @@ __global__ __launch_bounds__(256) void pos_bwd_kernel(const float* __restrict__ 
     const size_t base = static_cast<size_t>(t) * nv + j;
     fvec<W> acc = vload<W>(gpos, base);
     int b = 0;
-    for (; b + 4 <= batch; b += 4) {
-        fvec<W> q[4];
+    // Latency-bound at small seq * dim (a thread per vector, few threads):
+    // 8 rows per round trip instead of 4.
+    for (; b + 8 <= batch; b += 8) {
+        fvec<W> q[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) q[u] = vload<W>(g, base + (b + u) * row_stride);
+        for (int u = 0; u < 8; ++u) q[u] = vload<W>(g, base + (b + u) * row_stride);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < 8; ++u)
 #pragma unroll
             for (int e = 0; e < W; ++e) acc.v[e] = acc.v[e] + q[u].v[e];
     }
@@ -141,30 +143,60 @@ __global__ __launch_bounds__(256) void pos_bwd_kernel(const float* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Token backward, owner-computes form.  Workgroup k of K (a power of two)
-// owns the valid ids with id % K == k, so no two workgroups touch the same
-// table row.  Every workgroup reads the whole id vector (4 bytes per token,
-// served from L2, against 3 KB of grad row per token) and keeps the
-// positions of its own ids, in position order, in an LDS list (windows of
-// kOwnCap entries).  The list is sorted by id in LDS, stably, so that each
-// id's entries form a run in increasing position; the waves take runs from
-// an LDS counter and add each run onto its table row (one load, the run's
-// grad rows in order, one store).  Every row therefore receives its grad
-// rows in increasing token position, as in the CPU loop, and the result is
-// bit-identical whichever wave adds a run.  Measured at config 2 (16384
-// tokens, D = 768): 34 us against 46.7 us for a six-launch radix sort plus
-// an accumulate pass.
+// Token backward, owner-computes form.  The valid ids are split into K (a
+// power of two) classes, id % K, and each class belongs to S workgroups.
+// Every workgroup reads the whole id vector (4 bytes per token, served from
+// L2, against 3 KB of grad row per token) and keeps the positions of its
+// class's ids, in position order, in an LDS list, which is sorted by id in
+// LDS, stably, so that each id's entries form a run in increasing position.
+// Runs of at least kHeavy rows are added by the S workgroups together, each
+// its own slice of the columns (add_heavy); a shorter run is added by one wave
+// of one of them (one load of the table row, the run's grad rows in order,
+// one store).  Every element of a table row therefore receives its grad rows
+// in increasing token position, as in the CPU loop, and the result is
+// bit-identical whichever workgroup or wave adds it.
+//
+// What bounds it depends on the ids.  Uniform over a large vocabulary (16384
+// tokens, D = 768, V = 50257: fwd + bwd 53.3 us, 54.6 with one workgroup per
+// class and every run on one wave): the random 3 KB rows, after ~9 us of
+// scan and sort in which only the position rows stream.  Frequencies of text
+// on the same shape: the longest runs, 66 us against 208 us when one wave
+// added each (a memory round trip per two rows of a 466-row run).  A few
+// characters (32 x 256 tokens of 65 ids, D = 512): 23 us against 287 us.
 // ---------------------------------------------------------------------------
 constexpr int kOwnWaves = 8;
 constexpr int kOwnThreads = kOwnWaves * kWave;   // 512
 constexpr int kOwnPer = 32;                      // ids per thread per pass
-constexpr int kOwnGroups = kOwnPer / 4;          // 4-id groups per thread
-constexpr int kOwnSpan = kOwnThreads * kOwnPer;  // positions per pass
+constexpr int kOwnPerSmall = 8;                  // the same for small token counts
 constexpr int kOwnCap = 2048;                    // list entries per window
-constexpr int kOwnBatch = 2;                     // grad rows per group of loads
 constexpr int kOwnTake = 2;                      // sorted entries per claim
-constexpr int kOwnMaxK = 512;                    // owning workgroups, at most
-constexpr int kOwnTokens = 32;                   // tokens per owner, about
+constexpr int kOwnMaxGrid = 512;                 // workgroups, at most
+#ifndef MI_OWN_LOG2S
+#define MI_OWN_LOG2S 2
+#endif
+#ifndef MI_OWN_LIST
+#define MI_OWN_LIST 256
+#endif
+constexpr int kOwnList = MI_OWN_LIST;            // list entries a class should have, at most
+constexpr int kOwnLog2S = MI_OWN_LOG2S;          // log2 of the workgroups that share a class
+#ifndef MI_OWN_TOKENS
+#define MI_OWN_TOKENS 8
+#endif
+constexpr int kOwnTokens = MI_OWN_TOKENS;        // tokens per workgroup, at least
+#ifndef MI_OWN_HEAVY
+#define MI_OWN_HEAVY 16
+#endif
+constexpr int kHeavy = MI_OWN_HEAVY;             // rows of a run that the whole workgroup adds
+// Vectors per thread per staged batch of a long run (32 KB of LDS with 16-byte vectors, 16 KB with scalars).
+template <int W>
+constexpr int heavy_vecs() {
+    return W == 4 ? 4 : 8;
+}
+constexpr int kSlotBits = 11;                    // list slots fit: 2^11 = kOwnCap
+#ifndef MI_OWN_RANK
+#define MI_OWN_RANK 128
+#endif
+constexpr int kRankMax = MI_OWN_RANK;            // longest list sorted by rank
 
 // Position gradient fused into the owner kernel (POS): the workgroups also
 // share out the seq * nv position column vectors, one per thread per round;
@@ -179,55 +211,106 @@ constexpr int kPosPre = 7;   // batch rows in flight across the id scan, at most
 constexpr int kPosChunk = 5; // batch rows per group of loads afterwards
 
 // 128 VGPRs at most, so that two 8-wave workgroups fit on a CU.
-template <int W, int NCH, bool POS>
+template <int W, int NCH, int PER, bool POS>
 __global__ __launch_bounds__(kOwnThreads) __attribute__((amdgpu_waves_per_eu(4))) void
-emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids, int nblk,
+emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
                      const int* __restrict__ ids, const float* __restrict__ g,
                      float* __restrict__ table, float* __restrict__ gpos) {
-    __shared__ __align__(16) int s_id[kOwnCap];  // list in position order
-    __shared__ int s_pos[kOwnCap];
-    __shared__ int s_sid[kOwnCap];  // list sorted by id
-    __shared__ int s_spos[kOwnCap];
+    constexpr int kSpan = kOwnThreads * PER;       // positions per pass
+    // Grad rows per group of loads in a short run: as many as the registers
+    // of NCH column vectors per lane leave room for.
+    constexpr int kHeavyU = heavy_vecs<W>();
+    constexpr int kBins = kOwnThreads * kHeavyU * W / kOwnWaves;  // counts kept in s_stage
+    constexpr int kBatch = NCH == 1 ? 8 : NCH == 2 ? 4 : 2;
+    // The list: keys and positions, [0] in position order, sorted in [srt]
+    // (with room for the padding that the rank sort reads).  A key is the
+    // id's number within the class (id / K) with the list slot in its low
+    // bits, where it fits 32 bits so; no two keys are then equal, and their
+    // order is the stable order by id.
+    __shared__ __align__(16) unsigned s_keyb[2][kOwnCap + 16];
+    __shared__ int s_posb[2][kOwnCap];
     __shared__ int s_wsum[kOwnWaves];
-    __shared__ int s_next;
+    __shared__ int s_next, s_or, s_nheavy, s_nlight;
+    __shared__ int s_heavy[kOwnCap / kHeavy], s_hlen[kOwnCap / kHeavy];  // long runs
+    __shared__ __align__(16) float s_stage[kOwnThreads * kHeavyU * W];  // their staged rows
+    unsigned* const s_key = s_keyb[0];
+    int* const s_pos = s_posb[0];
+    int srt = 1;  // buffer that holds the sorted list
     __shared__ fvec<W> s_pacc[POS ? kOwnThreads : 1];  // first position rows, summed
     const int lane = threadIdx.x & (kWave - 1);
     // Uniform over the wave; readfirstlane lets the compiler see that, so
     // branches on it are scalar branches, not exec-masked ones.
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
-    // nblk (= gridDim.x, passed and preloaded with the other arguments) is a
-    // power of two, so id % nblk is a mask.
-    const unsigned kmask = static_cast<unsigned>(nblk) - 1u;
-    const unsigned k = blockIdx.x;
+    // cfg packs log2 K and log2 S (one preloaded argument).
+    const int log2k = cfg & 31;
+    const int log2s = cfg >> 5;
+    const int nblk = 1 << (log2k + log2s);
+    const unsigned k = blockIdx.x & ((1u << log2k) - 1u);
+    const int part = static_cast<int>(blockIdx.x >> log2k);
     const int nv = dim / W;
+    // An id of class k: rotating id ^ k right by log2 K leaves id / K, and a
+    // value of at least 2^(32 - log2 K) for the ids of other classes, so one
+    // unsigned compare with the number of this class's valid ids tests the
+    // class, the vocabulary bound and the sign together.
+    const unsigned vlim = vocab > 0 ? static_cast<unsigned>(vocab) : 0x80000000u;
+    const unsigned qlim = vlim > k ? ((vlim - 1u - k) >> log2k) + 1u : 0u;
+    auto number = [&](int id) __attribute__((always_inline)) {
+        const unsigned x = static_cast<unsigned>(id) ^ k;
+        return __builtin_amdgcn_alignbit(x, x, static_cast<unsigned>(log2k));
+    };
+    const int kshift = qlim <= (1u << (32 - kSlotBits)) - 1u ? kSlotBits : 0;
+    auto key_of = [&](unsigned num, int slot) __attribute__((always_inline)) {
+        return kshift != 0 ? (num << kSlotBits) | static_cast<unsigned>(slot) : num;
+    };
+    // The class number of a sorted entry, and the id it stands for.
+    auto num_at = [&](int e) __attribute__((always_inline)) { return s_keyb[srt][e] >> kshift; };
+    auto id_of = [&](unsigned num) __attribute__((always_inline)) {
+        return static_cast<size_t>((num << log2k) | k);
+    };
+    // This workgroup's column vectors of the long runs: slice `part` of S,
+    // whole 128-byte lines each (the last ones may be empty).
+    constexpr int kLine = 32 / W;
+    const int svec = (((nv + (1 << log2s) - 1) >> log2s) + kLine - 1) / kLine * kLine;
+    const int cbeg = part * svec;
+    const int cend = cbeg + svec < nv ? cbeg + svec : nv;
+
+    // Short runs: a workgroup adds whole rows ([lb, le) is [0, nv)) of the ids
+    // that are its own within the class.  Where a class fills its list more
+    // than once, an id's run may be long in one and short in the next, so
+    // every workgroup of the class then keeps to its column slice for the
+    // short runs too: each part of a table row has one workgroup that
+    // updates it, in list order.
+    bool sliced = false;
+    int lb = 0;
+    int le = nv;
 
     const unsigned long long below = (1ull << lane) - 1ull;
 
     // acc += the grad rows of sorted-list entries from, from + 1, ... while
-    // they carry `id` (none if entry `from` does not), in list order, for
-    // the column vectors c0 + lane + q * 64.
-    auto add_entries = [&](int id, int from, int L, int c0, fvec<W>(&acc)[NCH]) __attribute__((always_inline)) {
+    // they carry class number `num` (none if entry `from` does not), in list
+    // order, for the column vectors c0 + lane + q * 64.
+    auto add_entries = [&](unsigned num, int from, int L, int c0, fvec<W>(&acc)[NCH]) __attribute__((always_inline)) {
         for (int off = from;; off += kWave) {
             const int e = off + lane;
-            const bool same = e < L && s_sid[e] == id;
-            const int pos_l = same ? s_spos[e] : 0;
+            const bool same = e < L && num_at(e) == num;
+            const int pos_l = same ? s_posb[srt][e] : 0;
             const unsigned long long m = __ballot(same);
             const int cnt =
                 (~m == 0ull) ? kWave : (__ffsll(static_cast<unsigned long long>(~m)) - 1);
-            for (int u0 = 0; u0 < cnt; u0 += kOwnBatch) {
-                fvec<W> v[kOwnBatch][NCH];
+            for (int u0 = 0; u0 < cnt; u0 += kBatch) {
+                fvec<W> v[kBatch][NCH];
 #pragma unroll
-                for (int u = 0; u < kOwnBatch; ++u) {
+                for (int u = 0; u < kBatch; ++u) {
                     const int src = u0 + u < cnt ? u0 + u : 0;
                     const float* grow = g + static_cast<size_t>(__shfl(pos_l, src, kWave)) * dim;
 #pragma unroll
                     for (int q = 0; q < NCH; ++q) {
                         const int j = c0 + lane + q * kWave;
-                        v[u][q] = (u0 + u < cnt && j < nv) ? vload<W>(grow, j) : vzero<W>();
+                        v[u][q] = (u0 + u < cnt && j < le) ? vload<W>(grow, j) : vzero<W>();
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < kOwnBatch; ++u)
+                for (int u = 0; u < kBatch; ++u)
                     if (u0 + u < cnt) {
 #pragma unroll
                         for (int q = 0; q < NCH; ++q)
@@ -242,20 +325,20 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids,
     // Adds the run starting at sorted-list entry s0 (entries s0, s0 + 1, ...
     // with the id of s0, in position order) onto that id's table row.
     auto add_run = [&](int s0, int L) __attribute__((always_inline)) {
-        const int id = s_sid[s0];
-        float* row = table + static_cast<size_t>(id) * dim;
-        for (int c0 = 0; c0 < nv; c0 += NCH * kWave) {
+        const unsigned num = num_at(s0);
+        float* row = table + id_of(num) * dim;
+        for (int c0 = lb; c0 < le; c0 += NCH * kWave) {
             fvec<W> acc[NCH];
 #pragma unroll
             for (int q = 0; q < NCH; ++q) {
                 const int j = c0 + lane + q * kWave;
-                acc[q] = j < nv ? vload<W>(row, j) : vzero<W>();
+                acc[q] = j < le ? vload<W>(row, j) : vzero<W>();
             }
-            add_entries(id, s0, L, c0, acc);
+            add_entries(num, s0, L, c0, acc);
 #pragma unroll
             for (int q = 0; q < NCH; ++q) {
                 const int j = c0 + lane + q * kWave;
-                if (j < nv) vstore<W>(row, j, acc[q]);
+                if (j < le) vstore<W>(row, j, acc[q]);
             }
         }
     };
@@ -264,20 +347,20 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids,
     // two table rows and the first grad row of each run are requested at
     // once; the rest of each run (if any) follows.
     auto add_pair = [&](int sa, int sb, int L) __attribute__((always_inline)) {
-        const int ida = s_sid[sa];
-        const int idb = s_sid[sb];
-        float* ra = table + static_cast<size_t>(ida) * dim;
-        float* rb = table + static_cast<size_t>(idb) * dim;
-        const float* ga = g + static_cast<size_t>(s_spos[sa]) * dim;
-        const float* gb = g + static_cast<size_t>(s_spos[sb]) * dim;
-        for (int c0 = 0; c0 < nv; c0 += NCH * kWave) {
+        const unsigned na = num_at(sa);
+        const unsigned nb = num_at(sb);
+        float* ra = table + id_of(na) * dim;
+        float* rb = table + id_of(nb) * dim;
+        const float* ga = g + static_cast<size_t>(s_posb[srt][sa]) * dim;
+        const float* gb = g + static_cast<size_t>(s_posb[srt][sb]) * dim;
+        for (int c0 = lb; c0 < le; c0 += NCH * kWave) {
             fvec<W> A[NCH], B[NCH];
             {
                 fvec<W> GA[NCH], GB[NCH];
 #pragma unroll
                 for (int q = 0; q < NCH; ++q) {
                     const int j = c0 + lane + q * kWave;
-                    const bool ok = j < nv;
+                    const bool ok = j < le;
                     A[q] = ok ? vload<W>(ra, j) : vzero<W>();
                     B[q] = ok ? vload<W>(rb, j) : vzero<W>();
                     GA[q] = ok ? vload<W>(ga, j) : vzero<W>();
@@ -291,12 +374,12 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids,
                         B[q].v[x] = B[q].v[x] + GB[q].v[x];
                     }
             }
-            add_entries(ida, sa + 1, L, c0, A);
-            add_entries(idb, sb + 1, L, c0, B);
+            add_entries(na, sa + 1, L, c0, A);
+            add_entries(nb, sb + 1, L, c0, B);
 #pragma unroll
             for (int q = 0; q < NCH; ++q) {
                 const int j = c0 + lane + q * kWave;
-                if (j < nv) {
+                if (j < le) {
                     vstore<W>(ra, j, A[q]);
                     vstore<W>(rb, j, B[q]);
                 }
@@ -304,64 +387,380 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids,
         }
     };
 
-    // Sorts list entries [0, L) by id into s_sid / s_spos (a rank sort over
-    // 4-entry LDS reads; equal ids keep their position order).  The waves
-    // then take sorted entries from an LDS counter, one at a time, and the
-    // taker of an entry that starts a run of equal ids adds the whole run.
-    // Each run is added by one wave, whichever it is, so the result does
-    // not depend on the assignment.
+    // Adds the long runs (s_heavy / s_hlen) onto their table rows with the
+    // whole workgroup.  One wave adding such a run alone waits for a memory
+    // round trip per kBatch rows, which for the frequent ids of text
+    // (hundreds of rows per id) took longer than everything else; here the
+    // workgroup streams the rows through LDS, 512 * kHeavyU vectors per batch
+    // with two batches in flight in registers, and each thread adds the
+    // staged rows of one column in list order, so the sums are the ones a
+    // single wave would form, bit for bit.  The S workgroups of the class each
+    // add their own column slice, in chunks of 2^lcv vectors.  The batches of
+    // all chunks of all runs follow each other without a gap (run by run, a
+    // run of one batch took 5 us).
+    auto add_heavy = [&](int nheavy) __attribute__((always_inline)) {
+        int lcv = 3;
+        while (lcv < (W == 4 ? 6 : 8) && (1 << lcv) < cend - cbeg) ++lcv;
+        const int cv = 1 << lcv;
+        const int cw = cv * W;                                // columns per chunk
+        const int rpp = kOwnThreads >> lcv;                   // rows per vector of a thread
+        const int rb = rpp * kHeavyU;                         // rows per batch
+        const int vec = threadIdx.x & (cv - 1);
+        const int r0 = static_cast<int>(threadIdx.x) >> lcv;
+        const int col = static_cast<int>(threadIdx.x);
+        // Where the requests and the sums are: run h (entries s0 .. s0 + cnt),
+        // chunk from column vector c0, row b of the run.
+        struct At {
+            int h, s0, cnt, c0, b;
+            float* row;
+        };
+        auto enter = [&](At& a) __attribute__((always_inline)) {
+            a.s0 = __builtin_amdgcn_readfirstlane(s_heavy[a.h]);
+            a.cnt = __builtin_amdgcn_readfirstlane(s_hlen[a.h]);
+            a.row = table + id_of(static_cast<unsigned>(
+                                __builtin_amdgcn_readfirstlane(static_cast<int>(num_at(a.s0))))) *
+                                dim;
+            a.c0 = cbeg;
+            a.b = 0;
+        };
+        auto advance = [&](At& a) __attribute__((always_inline)) {
+            a.b += rb;
+            if (a.b >= a.cnt) {
+                a.b = 0;
+                a.c0 += cv;
+                if (a.c0 >= cend) {
+                    ++a.h;
+                    if (a.h < nheavy) enter(a);
+                }
+            }
+        };
+        At rq, su;
+        rq.h = 0;
+        enter(rq);
+        su = rq;
+        struct Batch {
+            fvec<W> v[kHeavyU];
+            float old;
+        };
+        // Loads are clamped into the run and the slice (past the last batch
+        // they repeat rows of the last run); only rows and columns in range
+        // are added.
+        auto request = [&](Batch& d) __attribute__((always_inline)) {
+            const int j = rq.c0 + vec < cend ? rq.c0 + vec : cend - 1;
+#pragma unroll
+            for (int u = 0; u < kHeavyU; ++u) {
+                const int r = rq.b + u * rpp + r0;
+                const int p = s_posb[srt][rq.s0 + (r < rq.cnt ? r : rq.cnt - 1)];
+                d.v[u] = vload<W>(g + static_cast<size_t>(p) * dim, j);
+            }
+            const int oc = rq.c0 * W + col;
+            d.old = rq.row[oc < cend * W ? oc : cend * W - 1];
+            advance(rq);
+        };
+        // A wave alone on its SIMD issues an instruction every 4 to 8 cycles,
+        // so the sums, one LDS read and one dependent add per row, are most
+        // of a batch's time; the row pitch is a constant so that the reads
+        // need no address arithmetic (30 cycles a row with it, 20 without).
+        // Only the last group may be partial (its reads stay in the batch).
+        auto sum_rows = [](float a, const float* p, int rows, auto pitch) __attribute__((always_inline)) {
+            constexpr int kPitch = decltype(pitch)::value;
+            for (int r = 0; r < rows; r += 16, p += 16 * kPitch) {
+                float x[16];
+#pragma unroll
+                for (int q = 0; q < 16; ++q) x[q] = p[q * kPitch];
+                if (r + 16 <= rows) {
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) a = a + x[q];
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) a = r + q < rows ? a + x[q] : a;
+                }
+            }
+            return a;
+        };
+        float cur = 0.0f;
+        auto consume_batch = [&](Batch& d) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < kHeavyU; ++u)
+                *reinterpret_cast<fvec<W>*>(&s_stage[((u * rpp + r0) * cv + vec) * W]) = d.v[u];
+            cur = su.b == 0 ? d.old : cur;
+            request(d);
+            __syncthreads();
+            if (su.h < nheavy) {
+                if (col < cw) {
+                    const int left = su.cnt - su.b;
+                    const int rows = left < rb ? left : rb;
+                    const float* p = s_stage + col;
+                    switch (lcv) {
+                        case 3: cur = sum_rows(cur, p, rows, std::integral_constant<int, 8 * W>{}); break;
+                        case 4: cur = sum_rows(cur, p, rows, std::integral_constant<int, 16 * W>{}); break;
+                        case 5: cur = sum_rows(cur, p, rows, std::integral_constant<int, 32 * W>{}); break;
+                        default:
+                            if constexpr (W == 4) {
+                                cur = sum_rows(cur, p, rows, std::integral_constant<int, 64 * W>{});
+                            } else {
+                                if (lcv == 6)
+                                    cur = sum_rows(cur, p, rows, std::integral_constant<int, 64>{});
+                                else if (lcv == 7)
+                                    cur = sum_rows(cur, p, rows, std::integral_constant<int, 128>{});
+                                else
+                                    cur = sum_rows(cur, p, rows, std::integral_constant<int, 256>{});
+                            }
+                    }
+                    const int oc = su.c0 * W + col;
+                    if (su.b + rb >= su.cnt && oc < cend * W) su.row[oc] = cur;
+                }
+                advance(su);
+            }
+            __syncthreads();
+        };
+        // In this order: swapped by the scheduler, the first batch's wait
+        // became a wait for both, in every trip of the loop.  All batches every
+        // time: with a batch conditional, the compiler waited for all
+        // outstanding loads before each one.
+        Batch A, B;
+        request(A);
+        __builtin_amdgcn_sched_barrier(0);
+        request(B);
+        __builtin_amdgcn_sched_barrier(0);
+        do {
+            consume_batch(A);
+            consume_batch(B);
+        } while (su.h < nheavy);
+    };
+
+    // Sorts list entries [0, L) by id, stably: lists of up to kRankMax
+    // entries by rank, four threads an entry (a list of 450 took 11 us that
+    // way), longer ones by counting where a class has at most kBins ids, else
+    // by radix, one of the id bits that differ per pass (9 us for 9 bits).  Runs of at least kHeavy rows are
+    // added by the class's workgroups together, by column slices; of the
+    // shorter runs a workgroup takes those whose id / K mod S is its number,
+    // and its waves share them out through an LDS counter.  Each run is added
+    // in position order whoever adds it, so the result does not depend on
+    // the assignment.
     auto process = [&](int L) __attribute__((always_inline)) {
-        for (int i = static_cast<int>(threadIdx.x); i < L; i += kOwnThreads) {
-            const int me = s_id[i];
-            int r = 0;
-            int j = 0;
-            for (; j + 4 <= L; j += 4) {
-                const int4 o = *reinterpret_cast<const int4*>(&s_id[j]);
-                r += (o.x < me || (o.x == me && j < i)) ? 1 : 0;
-                r += (o.y < me || (o.y == me && j + 1 < i)) ? 1 : 0;
-                r += (o.z < me || (o.z == me && j + 2 < i)) ? 1 : 0;
-                r += (o.w < me || (o.w == me && j + 3 < i)) ? 1 : 0;
-            }
-            for (; j < L; ++j) {
-                const int o = s_id[j];
-                r += (o < me || (o == me && j < i)) ? 1 : 0;
-            }
-            s_sid[r] = me;
-            s_spos[r] = s_pos[i];
+        if (threadIdx.x == 0) {
+            s_next = 0;
+            s_nheavy = 0;
+            s_nlight = 0;
         }
-        if (threadIdx.x == 0) s_next = 0;
+        if (kshift != 0 && L <= kRankMax) {
+            srt = 1;
+            if (threadIdx.x < 16) s_key[L + threadIdx.x] = 0xffffffffu;
+            __syncthreads();
+            const int sub = static_cast<int>(threadIdx.x) & 3;
+            for (int i0 = 0; i0 < L; i0 += kOwnThreads / 4) {
+                const int i = i0 + (static_cast<int>(threadIdx.x) >> 2);
+                if (i0 + wave * (kWave / 4) >= L) break;  // wave-uniform
+                const unsigned me = s_key[i < L ? i : 0];
+                int r = 0;
+#pragma unroll 4
+                for (int j = 4 * sub; j < L; j += 16) {
+                    const uint4 o = *reinterpret_cast<const uint4*>(&s_key[j]);
+                    r += (o.x < me) + (o.y < me) + (o.z < me) + (o.w < me);
+                }
+                r += __shfl_xor(r, 1, kWave);
+                r += __shfl_xor(r, 2, kWave);
+                if (i < L) {
+                    if (sub == 0) s_keyb[1][r] = me;
+                    if (sub == 1) s_posb[1][r] = s_pos[i];
+                }
+            }
+        } else if (qlim <= kBins) {
+            // Wave w holds entries w * span + [0, span) in groups of 64.  A
+            // group's lanes find the lanes of the same number from one ballot
+            // per bit; an entry's place among its number's entries is the
+            // wave's count before the group plus the equal lanes below it.
+            // The counts of all waves, summed over the waves and then over
+            // the numbers, give every (wave, number) its first slot.
+            constexpr int kQ = kOwnCap / kOwnThreads;
+            const int span = (L + kOwnThreads - 1) / kOwnThreads * kWave;
+            int* const cnt = reinterpret_cast<int*>(s_stage);  // [wave][kBins]
+            const int nbin = static_cast<int>(qlim);
+            const int nbits = 32 - __builtin_clz(static_cast<unsigned>(nbin) | 1u);
+            for (int i = static_cast<int>(threadIdx.x); i < kOwnWaves * kBins; i += kOwnThreads)
+                cnt[i] = 0;
+            __syncthreads();
+            unsigned me[kQ];
+            int at[kQ];
+#pragma unroll
+            for (int q = 0; q < kQ; ++q) {
+                if (q * kWave >= span) break;  // uniform
+                const int i = wave * span + q * kWave + lane;
+                const bool ok = i < L;
+                me[q] = ok ? s_key[i] : 0u;
+                const unsigned num = me[q] >> kshift;
+                unsigned long long same = __ballot(ok);
+                for (int b = 0; b < nbits; ++b) {
+                    const bool bit = ((num >> b) & 1u) != 0;
+                    const unsigned long long m = __ballot(bit);
+                    same &= bit ? m : ~m;
+                }
+                if (ok) {
+                    int* const c = &cnt[wave * kBins + static_cast<int>(num)];
+                    at[q] = *c + __popcll(same & below);
+                    if ((same & below) == 0ull) *c += __popcll(same);
+                }
+            }
+            __syncthreads();
+            // Thread t takes the numbers t * kPer + [0, kPer).
+            constexpr int kPer = kBins / kOwnThreads;
+            int bsum = 0;
+#pragma unroll
+            for (int b = 0; b < kPer; ++b)
+#pragma unroll
+                for (int w = 0; w < kOwnWaves; ++w)
+                    bsum += cnt[w * kBins + static_cast<int>(threadIdx.x) * kPer + b];
+            int upto = bsum;  // inclusive sum over the wave's lanes
+#pragma unroll
+            for (int o = 1; o < kWave; o *= 2) {
+                const int v = __shfl_up(upto, o, kWave);
+                upto += lane >= o ? v : 0;
+            }
+            if (lane == kWave - 1) s_wsum[wave] = upto;
+            __syncthreads();
+            int run = upto - bsum;
+#pragma unroll
+            for (int w = 0; w < kOwnWaves; ++w) run += w < wave ? s_wsum[w] : 0;
+#pragma unroll
+            for (int b = 0; b < kPer; ++b)
+#pragma unroll
+                for (int w = 0; w < kOwnWaves; ++w) {
+                    int* const c = &cnt[w * kBins + static_cast<int>(threadIdx.x) * kPer + b];
+                    const int v = *c;
+                    *c = run;
+                    run += v;
+                }
+            __syncthreads();
+            srt = 1;
+#pragma unroll
+            for (int q = 0; q < kQ; ++q) {
+                if (q * kWave >= span) break;
+                const int i = wave * span + q * kWave + lane;
+                if (i < L) {
+                    const int to = cnt[wave * kBins + static_cast<int>(me[q] >> kshift)] + at[q];
+                    s_keyb[1][to] = me[q];
+                    s_posb[1][to] = s_pos[i];
+                }
+            }
+        } else {
+            // Wave w holds entries w * span + [0, span) in groups of 64; a
+            // pass moves the entries with a 0 bit in front of those with a 1
+            // bit, both in list order.
+            constexpr int kQ = kOwnCap / kOwnThreads;
+            const int span = (L + kOwnThreads - 1) / kOwnThreads * kWave;
+            const unsigned first = s_key[0];
+            if (threadIdx.x == 0) s_or = 0;
+            __syncthreads();
+            unsigned diff = 0;
+            for (int i = static_cast<int>(threadIdx.x); i < L; i += kOwnThreads)
+                diff |= s_key[i] ^ first;
+            diff = diff >> kshift << kshift;
+            if (diff != 0) atomicOr(&s_or, static_cast<int>(diff));
+            __syncthreads();
+            unsigned todo = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(s_or));
+            srt = 0;
+            while (todo != 0) {
+                const int bit = __ffs(static_cast<int>(todo)) - 1;
+                todo &= todo - 1;
+                unsigned me[kQ];
+                int zero_before[kQ], mp[kQ];
+                int zeros = 0;
+#pragma unroll
+                for (int q = 0; q < kQ; ++q) {
+                    if (q * kWave >= span) break;  // uniform
+                    const int i = wave * span + q * kWave + lane;
+                    me[q] = i < L ? s_keyb[srt][i] : 0u;
+                    mp[q] = i < L ? s_posb[srt][i] : 0;
+                    const unsigned long long z = __ballot(i < L && !((me[q] >> bit) & 1u));
+                    zero_before[q] = zeros + __popcll(z & below);
+                    zeros += __popcll(z);
+                }
+                if (lane == 0) s_wsum[wave] = zeros;
+                __syncthreads();
+                int zb = 0, zt = 0;
+#pragma unroll
+                for (int w = 0; w < kOwnWaves; ++w) {
+                    const int t = s_wsum[w];
+                    zb += w < wave ? t : 0;
+                    zt += t;
+                }
+#pragma unroll
+                for (int q = 0; q < kQ; ++q) {
+                    if (q * kWave >= span) break;
+                    const int i = wave * span + q * kWave + lane;
+                    const int z = zb + zero_before[q];  // zeros in front of entry i
+                    const int to = ((me[q] >> bit) & 1u) ? zt + i - z : z;
+                    if (i < L) {
+                        s_keyb[srt ^ 1][to] = me[q];
+                        s_posb[srt ^ 1][to] = mp[q];
+                    }
+                }
+                srt ^= 1;
+                __syncthreads();
+            }
+        }
         __syncthreads();
+        // The runs: long ones into s_heavy, this workgroup's short ones into
+        // the key buffer that the sort has left free.
+        unsigned* const s_light = s_keyb[srt ^ 1];
+        for (int i0 = 0; i0 < L; i0 += kOwnThreads) {
+            const int i = i0 + static_cast<int>(threadIdx.x);
+            const unsigned me = i < L ? num_at(i) : 0u;
+            const bool start = i < L && (i == 0 || num_at(i - 1) != me);
+            const bool heavy = start && i + kHeavy <= L && num_at(i + kHeavy - 1) == me;
+            if (heavy) {
+                int lo = i + kHeavy, hi = L;  // end of the run in [lo, hi]
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (num_at(mid) == me)
+                        lo = mid + 1;
+                    else
+                        hi = mid;
+                }
+                const int slot = atomicAdd(&s_nheavy, 1);
+                s_heavy[slot] = i;
+                s_hlen[slot] = lo - i;
+            }
+            const bool light =
+                start && !heavy &&
+                (sliced || static_cast<int>(me & ((1u << log2s) - 1u)) == part);
+            const unsigned long long m = __ballot(light);
+            int at = 0;
+            if (lane == 0 && m != 0) at = atomicAdd(&s_nlight, static_cast<int>(__popcll(m)));
+            at = __shfl(at, 0, kWave);
+            if (light) s_light[at + __popcll(m & below)] = static_cast<unsigned>(i);
+        }
+        __syncthreads();
+        if (cbeg < cend) {
+            const int nheavy = __builtin_amdgcn_readfirstlane(s_nheavy);
+            if (nheavy > 0) add_heavy(nheavy);
+        }
+        const int nlight = s_nlight;
         for (;;) {
             int e = 0;
             if (lane == 0) e = atomicAdd(&s_next, kOwnTake);
             e = __shfl(e, 0, kWave);
-            if (e >= L) break;
-            const bool sa = e == 0 || s_sid[e - 1] != s_sid[e];
-            const bool sb = kOwnTake == 2 && e + 1 < L && s_sid[e] != s_sid[e + 1];
-            if (sa && sb)
-                add_pair(e, e + 1, L);
-            else if (sa)
-                add_run(e, L);
-            else if (sb)
-                add_run(e + 1, L);
+            if (e >= nlight) break;
+            if (kOwnTake == 2 && e + 1 < nlight)
+                add_pair(static_cast<int>(s_light[e]), static_cast<int>(s_light[e + 1]), L);
+            else
+                add_run(static_cast<int>(s_light[e]), L);
         }
     };
 
     // Position gradient, first round: requests issued now, summed below.
     const long long pvec = POS ? static_cast<long long>(seq) * nv : 0;   // position vectors
     const long long pstride = static_cast<long long>(nblk) * kOwnThreads;
-    // A thread's first position vector, below kOwnMaxK * kOwnThreads = 2^18:
+    // A thread's first position vector, below kOwnMaxGrid * kOwnThreads = 2^18:
     // 32 bits.  Held as a 64-bit value it was spilled to scratch, and its
     // reload waited for every outstanding load.
-    const int pv0 = static_cast<int>(k) * kOwnThreads + wave * kWave + lane;
+    const int pv0 = static_cast<int>(blockIdx.x) * kOwnThreads + wave * kWave + lane;
     const size_t bstride = static_cast<size_t>(seq) * nv;                // vectors per batch row
     // PRE batch rows of the first position vector are requested across the
     // id scan (7 for 2-3 column vectors per lane, 4 for one: more spills
-    // registers in the scan); with 4 column vectors per lane none fit, and the
-    // position sums run after the token gradient alone.  The position
-    // bookkeeping kept across the token updates stays in registers (no
-    // instantiation spills).
-    constexpr int PRE = !POS ? 0 : NCH == 1 ? 4 : NCH <= 3 ? kPosPre : 0;
+    // registers in the scan).
+    constexpr int PRE = !POS ? 0 : NCH == 1 ? 4 : kPosPre;
     constexpr int NPQ = PRE > 0 ? PRE : 1;
     // Adds batch rows b0, b0 + 1, ... of position vector pv onto acc, in
     // order, and stores the total.
@@ -385,49 +784,38 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids,
             pos_rest(pv, 0, vload<W>(gpos, pv));
     };
 
-    // One pass over kOwnSpan positions of the id vector.  The first pass is
-    // a separate instantiation (FIRST) so that the position registers live
-    // only inside it.  This lambda and those it calls are inlined: an
-    // out-of-line call keeps the captured locals in scratch memory.
-    auto pass = [&](long long base, auto first_tag) __attribute__((always_inline)) {
+    // One scan of kSpan positions of the id vector: this class's ids are
+    // appended to the list, behind the `filled` entries that it holds, if they
+    // all fit; `total` says how many there are.  The first scan is a separate
+    // instantiation (FIRST) so that the position registers live only inside
+    // it.  This lambda and those it calls are inlined: an out-of-line call
+    // keeps the captured locals in scratch memory.
+    int filled = 0, total = 0, before = 0;
+    unsigned wpos = 0;
+    const unsigned un = static_cast<unsigned>(n);
+    auto scan = [&](unsigned base, auto first_tag) __attribute__((always_inline)) {
         constexpr bool first = decltype(first_tag)::value && PRE > 0;
         [[maybe_unused]] fvec<W> pacc, pq[NPQ];
-        // Wave w reads positions base + w * kOwnPer * 64 + [0, kOwnPer * 64):
-        // group j (4 ids per lane) covers 256 consecutive positions, lane l
-        // takes positions 4l .. 4l + 3 of it, so every load instruction of
-        // the wave reads one contiguous KiB.  bits marks the ids this
-        // workgroup owns.
-        const long long wpos = base + static_cast<long long>(wave) * kOwnPer * kWave;
-        int my[kOwnPer];
-        unsigned bits = 0;
-        // Either the wave's whole span is in range with 16-byte aligned ids
-        // (one 16-byte load per group) or every id is a 4-byte load at a
-        // clamped position, masked after the load.  The choice is uniform
-        // over the wave and no load sits under a per-lane branch, so the
-        // waits that follow count these loads exactly: with per-lane
-        // branches the compiler waited for all but one of the position loads
-        // issued below before the first id was tested, which serialised
-        // them with the scan.
-        if (vec_ids && wpos + kOwnPer * kWave <= n) {
+        // Wave w reads positions base + w * PER * 64 + [0, PER * 64), load e
+        // of lane l position 64 e + l of it: list order is load order, then
+        // lane order, and every load instruction of the wave reads 256
+        // contiguous bytes.
+        wpos = base + static_cast<unsigned>(wave) * PER * kWave;
+        int my[PER];
+        // The choice is uniform over the wave and no load sits under a
+        // per-lane branch, so the waits that follow count these loads
+        // exactly: with per-lane branches the compiler waited for all but
+        // one of the position loads issued below before the first id was
+        // tested, which serialised them with the scan.
+        if (wpos + PER * kWave <= un) {
 #pragma unroll
-            for (int j = 0; j < kOwnGroups; ++j) {
-                const long long p4 = wpos + j * 4 * kWave + 4 * lane;
-                const int4 v = *reinterpret_cast<const int4*>(ids + p4);
-                my[4 * j] = v.x;
-                my[4 * j + 1] = v.y;
-                my[4 * j + 2] = v.z;
-                my[4 * j + 3] = v.w;
-            }
+            for (int e = 0; e < PER; ++e) my[e] = ids[wpos + e * kWave + lane];
         } else {
 #pragma unroll
-            for (int j = 0; j < kOwnGroups; ++j) {
-                const long long p4 = wpos + j * 4 * kWave + 4 * lane;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const long long p = p4 + e;
-                    const int v = ids[p < n ? p : n - 1];
-                    my[4 * j + e] = p < n ? v : -1;
-                }
+            for (int e = 0; e < PER; ++e) {
+                const unsigned p = wpos + e * kWave + lane;
+                const int v = ids[p < un ? p : un - 1u];
+                my[e] = p < un ? v : -1;
             }
         }
         if constexpr (first) {
@@ -446,63 +834,44 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids,
                 pq[u] = sload<W>(g, static_cast<size_t>(u < batch ? u : batch - 1) * bstride +
                                         static_cast<size_t>(pvc));
         }
-#pragma unroll
-        for (int j = 0; j < kOwnGroups; ++j) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int id = my[4 * j + e];
-                const bool ok = id >= 0 && (vocab <= 0 || id < vocab) &&
-                                (static_cast<unsigned>(id) & kmask) == k;
-                bits |= static_cast<unsigned>(ok) << (4 * j + e);
-            }
-        }
-        // List slots in position order: within the wave from ballots
-        // (group, then lane, then element), across waves from their totals.
-        int lane_off[kOwnGroups];
+        // List slots in position order: the wave's matches are counted, its
+        // first slot comes from the other waves' counts, and a second look at
+        // the ids (in registers, three instructions each) writes them.
         int wtot = 0;
 #pragma unroll
-        for (int j = 0; j < kOwnGroups; ++j) {
-            int pre = 0, tot = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const unsigned long long b = __ballot((bits >> (4 * j + e)) & 1u);
-                pre += __popcll(b & below);
-                tot += __popcll(b);
-            }
-            lane_off[j] = wtot + pre;
-            wtot += tot;
-        }
+        for (int e = 0; e < PER; ++e) wtot += __popcll(__ballot(number(my[e]) < qlim));
         if (lane == 0) s_wsum[wave] = wtot;
         __syncthreads();
-        int before = 0, total = 0;
+        before = 0;
+        total = 0;
 #pragma unroll
         for (int w = 0; w < kOwnWaves; ++w) {
             const int t = s_wsum[w];
             before += w < wave ? t : 0;
             total += t;
         }
-        __syncthreads();  // s_wsum is rewritten by the next pass
-        // Windows of kOwnCap list entries (one window unless this
-        // workgroup's ids are very frequent in this span).  The first window
-        // is written from the ids in registers; later windows read their ids
-        // again, one at a time, so that no id registers stay live while the
-        // windows are processed.
-        if (total > 0) {
+        before = __builtin_amdgcn_readfirstlane(before);
+        total = __builtin_amdgcn_readfirstlane(total);
+        __syncthreads();  // s_wsum is rewritten later
+        const bool fits = filled + total <= kOwnCap;
+        if (fits && wtot > 0) {
+            int at = filled + before;
 #pragma unroll
-            for (int j = 0; j < kOwnGroups; ++j) {
-                int slot = before + lane_off[j];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if ((bits >> (4 * j + e)) & 1u) {
-                        if (slot < kOwnCap) {
-                            s_id[slot] = my[4 * j + e];
-                            s_pos[slot] = static_cast<int>(wpos + j * 4 * kWave + 4 * lane + e);
-                        }
-                        ++slot;
+            for (int e = 0; e < PER; ++e) {
+                const unsigned num = number(my[e]);
+                const bool ok = num < qlim;
+                const unsigned long long m = __ballot(ok);
+                if (m != 0) {
+                    const int slot = at + __popcll(m & below);
+                    if (ok) {
+                        s_key[slot] = key_of(num, slot);
+                        s_pos[slot] = static_cast<int>(wpos + e * kWave + lane);
                     }
+                    at += __popcll(m);
                 }
             }
         }
+        if (fits) filled += total;
         if constexpr (first) {
             if (pv0 < pvec) {
 #pragma unroll
@@ -513,34 +882,62 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int vec_ids,
                 s_pacc[threadIdx.x] = pacc;  // finished after the token gradient
             }
         }
-        for (int w0 = 0; w0 < total; w0 += kOwnCap) {
-            if (w0 > 0) {
+        return fits;
+    };
+    // Entries [w0, w0 + kOwnCap) of the span last scanned into the empty
+    // list, the ids read again one at a time (rare: the list was full, or one
+    // span holds more of the class's ids than a list does).
+    auto refill = [&](int w0) __attribute__((always_inline)) {
+        int at = before;
 #pragma unroll 1
-                for (int j = 0; j < kOwnGroups; ++j) {
-                    int slot = before + lane_off[j];
-#pragma unroll 1
-                    for (int e = 0; e < 4; ++e) {
-                        if ((bits >> (4 * j + e)) & 1u) {
-                            if (slot >= w0 && slot < w0 + kOwnCap) {
-                                const long long p = wpos + j * 4 * kWave + 4 * lane + e;
-                                s_id[slot - w0] = ids[p];
-                                s_pos[slot - w0] = static_cast<int>(p);
-                            }
-                            ++slot;
-                        }
-                    }
-                }
+        for (int e = 0; e < PER; ++e) {
+            const unsigned p = wpos + e * kWave + lane;
+            const unsigned num = number(p < un ? ids[p] : -1);
+            const bool ok = num < qlim;
+            const unsigned long long m = __ballot(ok);
+            const int slot = at + __popcll(m & below) - w0;
+            if (ok && slot >= 0 && slot < kOwnCap) {
+                s_key[slot] = key_of(num, slot);
+                s_pos[slot] = static_cast<int>(p);
             }
-            __syncthreads();
-            process(total - w0 < kOwnCap ? total - w0 : kOwnCap);
-            __syncthreads();
+            at += __popcll(m);
         }
     };
-    if constexpr (PRE > 0) {
-        pass(0, std::true_type{});
-        for (long long base = kOwnSpan; base < n; base += kOwnSpan) pass(base, std::false_type{});
-    } else {
-        for (long long base = 0; base < n; base += kOwnSpan) pass(base, std::false_type{});
+    // Scan spans until the list is full or the ids are done, then add the
+    // list's runs.  All of this is uniform over the workgroup, and the same
+    // for every workgroup of a class.
+    bool over = !scan(0u, std::true_type{});
+    unsigned base = 0;
+    int w0 = 0;
+    for (bool done = false; !done;) {
+        bool flush = true;
+        if (over && filled == 0) {
+            refill(w0);
+            filled = total - w0 < kOwnCap ? total - w0 : kOwnCap;
+            w0 += filled;
+            over = w0 < total;
+            flush = over;
+        } else if (!over) {
+            if (un - base > static_cast<unsigned>(kSpan)) {
+                base += kSpan;
+                over = !scan(base, std::false_type{});
+                w0 = 0;
+                flush = false;
+            } else {
+                done = true;
+            }
+        }
+        if (flush && filled > 0) {
+            if (!done) {
+                sliced = true;
+                lb = cbeg;
+                le = cend;
+            }
+            __syncthreads();
+            process(filled);
+            __syncthreads();
+            filled = 0;
+        }
     }
     // The rest of the position sums follow the token gradient: the table-row
     // updates start as soon as the list is built (config-2 step 58.8 ->
@@ -590,37 +987,50 @@ void launch_emb_fwd(const float* table, const float* pos, const int* tokens, flo
 #undef MI_FWD_CASE
 }
 
-// One launch of the owner kernel: K = 2^log2k owning workgroups, about
-// kOwnTokens tokens each.  The position gradient (POS) needs 16-byte
-// alignment of grad_pos as well for the vector path.
+// One launch of the owner kernel: a grid of 2^want workgroups, at least
+// kOwnTokens tokens each, as K = 2^log2k id classes of S = 2^log2s
+// workgroups.  S is 4, less where a class would then have more than kOwnList
+// tokens on average (a longer list takes longer to sort), and more where the
+// vocabulary has fewer ids than that leaves classes (characters, bytes).  The position gradient (POS) needs
+// 16-byte alignment of grad_pos as well for the vector path.
 template <bool POS>
 void launch_owner(const float* grad_out, const int* tokens, float* grad_table, float* grad_pos,
                   int batch_seq, int batch, int seq, int dim, int vocab, hipStream_t st) {
-    int log2k = 0;
-    while ((2 << log2k) <= kOwnMaxK && (2ll << log2k) * kOwnTokens <= batch_seq) ++log2k;
-    const dim3 grid(1u << log2k), block(kOwnThreads);
-    const bool vec_ids = aligned16(tokens);
     const bool v4 = dim % 4 == 0 && aligned16(grad_out) && aligned16(grad_table) &&
                     (!POS || aligned16(grad_pos));
+    int want = 0;
+    while ((2 << want) <= kOwnMaxGrid && (2ll << want) * kOwnTokens <= batch_seq) ++want;
+    int log2k = want > kOwnLog2S ? want - kOwnLog2S : 0;
+    while (log2k < want && (batch_seq >> log2k) > kOwnList) ++log2k;
+    if (vocab > 0)
+        while (log2k > 0 && (1 << log2k) > vocab) --log2k;
+    const int log2s = want - log2k;
+    const dim3 grid(1u << want), block(kOwnThreads);
+    const int cfg = log2k | (log2s << 5);
     const int nv = v4 ? dim / 4 : dim;
-    // Column vectors per lane held at once: just enough for the row, at most
-    // 4 (wider rows loop over column chunks).
-    const int nch = nv <= kWave ? 1 : nv <= 2 * kWave ? 2 : nv <= 3 * kWave ? 3 : 4;
-#define MI_OWNER_CASE(WW, NN)                                                                  \
-    hipLaunchKernelGGL((emb_bwd_owner_kernel<WW, NN, POS>), grid, block, 0, st, batch_seq,    \
-                       vocab, dim, batch, seq, vec_ids ? 1 : 0, 1 << log2k, tokens, grad_out, \
-                       grad_table, grad_pos)
+    // Column vectors per lane held at once, at most 3: the fewest that cover
+    // the row in as few column chunks.
+    const int chunks = (nv + 3 * kWave - 1) / (3 * kWave);
+    const int nch = (nv + chunks * kWave - 1) / (chunks * kWave);
+    const bool small = batch_seq <= kOwnThreads * kOwnPerSmall;
+#define MI_OWNER_LAUNCH(WW, NN, PP)                                                            \
+    hipLaunchKernelGGL((emb_bwd_owner_kernel<WW, NN, PP, POS>), grid, block, 0, st, batch_seq, \
+                       vocab, dim, batch, seq, cfg, tokens, grad_out, grad_table, grad_pos)
+#define MI_OWNER_CASE(WW, NN)                       \
+    if (small)                                      \
+        MI_OWNER_LAUNCH(WW, NN, kOwnPerSmall);      \
+    else                                            \
+        MI_OWNER_LAUNCH(WW, NN, kOwnPer)
     switch ((v4 ? 10 : 0) + nch) {
         case 11: MI_OWNER_CASE(4, 1); break;
         case 12: MI_OWNER_CASE(4, 2); break;
         case 13: MI_OWNER_CASE(4, 3); break;
-        case 14: MI_OWNER_CASE(4, 4); break;
         case 1: MI_OWNER_CASE(1, 1); break;
         case 2: MI_OWNER_CASE(1, 2); break;
-        case 3: MI_OWNER_CASE(1, 3); break;
-        default: MI_OWNER_CASE(1, 4); break;
+        default: MI_OWNER_CASE(1, 3); break;
     }
 #undef MI_OWNER_CASE
+#undef MI_OWNER_LAUNCH
 }
 
 }  // namespace

@@ -228,3 +228,50 @@ def test_embedding_backward_unaligned_ids_and_rows(dev, V, D, B, T, id_off, g_of
     Twte = dev_t(dwte0)
     M.embedding_backward(G, Ids, Twte, BT, D, V)
     assert_exact("token dwte, unaligned", host(Twte), O.embedding_backward(g, ids, dwte0))
+
+
+def _runs(lengths, vocab, n, seed):
+    """n ids: id 3 + 5 i occurs lengths[i] times, the rest is uniform; shuffled."""
+    r = np.random.default_rng(seed)
+    ids = [np.full(c, (3 + 5 * i) % vocab) for i, c in enumerate(lengths)]
+    left = n - sum(lengths)
+    ids.append(r.integers(0, vocab, left))
+    return r.permutation(np.concatenate(ids)).astype(np.int32)
+
+
+@pytest.mark.parametrize("V,D,n,lengths,vocab_arg", [
+    # run lengths around the shared-run threshold (16) and a staged batch
+    (5000, 768, 2000, (15, 16, 17, 31, 32, 33, 64, 65), 5000),
+    (5000, 100, 4096, (15, 16, 17, 128, 129, 300), 5000),   # slices of 25 vectors; last small span
+    (5000, 130, 4097, (16, 129, 257, 700), 5000),           # scalar columns; first large span
+    (5000, 36, 16384, (2040, 1500, 600, 40), 5000),         # a list near its capacity
+    (65, 512, 8192, (900, 800, 17), 65),                    # few ids: many slices per class
+    (65, 40, 16385, (5000, 300), 65),                       # empty last slices, list overflow
+    (3, 1030, 700, (300, 20), 3),                           # scalar columns, 5 column chunks
+    (70000, 16, 9000, (200, 150, 16), 0),                   # trusted ids: radix sort
+    (60000, 32, 60000, (3000, 2100, 500, 16), 60000),       # several scans into one list
+])
+def test_embedding_backward_run_lengths(dev, V, D, n, lengths, vocab_arg):
+    note(f"embedding runs V={V} D={D} n={n} lengths={lengths} vocab_arg={vocab_arg}")
+    r = np.random.default_rng(n + D)
+    ids = _runs(lengths, V, n, D)
+    g = r.standard_normal((n, D), dtype=np.float32)
+    dwte0 = r.standard_normal((V, D), dtype=np.float32)
+    dwpe0 = r.standard_normal((n, D), dtype=np.float32)
+    G, Ids, Dwte, Fwte, Fwpe = dev_t(g), dev_t(ids), dev_t(dwte0), dev_t(dwte0), dev_t(dwpe0)
+    expect = O.embedding_backward(g, ids, dwte0)
+    M.embedding_backward(G, Ids, Dwte, n, D, vocab_arg)
+    assert_exact("dwte", host(Dwte), expect)
+    M.embedding_pos_backward(G, Ids, Fwte, Fwpe, 1, n, D, vocab_arg)
+    assert_exact("fused dwte", host(Fwte), expect)
+    assert_exact("fused dwpe", host(Fwpe), O.pos_embedding_backward(g, dwpe0, 1, n))
+
+
+@pytest.mark.parametrize("B,T,D", [(1, 3, 5), (7, 5, 64), (8, 4, 64), (9, 4, 128), (17, 3, 33)])
+def test_pos_embedding_backward_batch_groups(dev, B, T, D):
+    r = np.random.default_rng(B)
+    g = r.standard_normal((B * T, D), dtype=np.float32)
+    dwpe0 = r.standard_normal((T, D), dtype=np.float32)
+    Dwpe = dev_t(dwpe0)
+    M.pos_embedding_backward(dev_t(g), Dwpe, B, T, D)
+    assert_exact("dwpe", host(Dwpe), O.pos_embedding_backward(g, dwpe0, B, T))
