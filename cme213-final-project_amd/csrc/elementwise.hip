@@ -309,6 +309,96 @@ __global__ __launch_bounds__(1024) void rowband_kernel(const void* w0, const voi
     }
 }
 
+// ---------------------------------------------------------------------------
+// Row-lane kernels: the reducing operators on narrow rows, and on rows whose
+// width is no multiple of 4.
+//
+// A row band of one row per workgroup leaves most of the chip idle on narrow
+// rows (one or two waves per CU at 256 or 512 columns: ReLU backward + dbias
+// [8192, 2048] 33 us, [2048, 512] 7.4 us) and falls back to 4-byte accesses
+// where rows do not start on 16 bytes.  Here a workgroup takes RL consecutive
+// rows at a time as one contiguous run of sv = RL * cols / 4 vectors, RL a
+// multiple of 4 / gcd(cols, 4), so that every run starts on 16 bytes: thread
+// t owns the super-columns of vectors t + k * T, keeps their biases and sums
+// in registers, and a vector may span two rows.  At the end the RL sums of
+// each column are added through LDS in row-lane order and the workgroup
+// writes one partial row, as a band does.  The at most 3 elements past the
+// last whole vector are the last row's: workgroup 0 takes them one by one.
+// ---------------------------------------------------------------------------
+template <int NC, class Op, class Op1>
+__global__ __launch_bounds__(1024) void rowlane_kernel(const void* w0, const void* w1,
+                                                       const void* w2,
+                                                       const float* __restrict__ bias,
+                                                       unsigned long long nvec, int sv, int T,
+                                                       int cols, int G, int tail,
+                                                       float* __restrict__ part) {
+    extern __shared__ __align__(16) float lane_sums[];  // [4 * sv], then tail values [4]
+    const Op op = op_from<Op>(w0, w1, w2);
+    fvec<4> bv[NC], acc[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const int j = threadIdx.x + k * T;
+        bv[k] = vzero<4>();
+        acc[k] = vzero<4>();
+        if (bias && j < sv) {
+            int c = static_cast<int>(4u * static_cast<unsigned>(j) % static_cast<unsigned>(cols));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                bv[k].v[e] = bias[c];
+                c = c + 1 == cols ? 0 : c + 1;
+            }
+        }
+    }
+    using In = typename Op::In;
+    const unsigned long long step = static_cast<unsigned long long>(G) * sv;
+    for (unsigned long long base = static_cast<unsigned long long>(blockIdx.x) * sv; base < nvec;
+         base += step) {
+        // Loads are unconditional, at clamped indices, and consumed before
+        // the first store, as in the row bands.
+        In in[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const int j = threadIdx.x + k * T;
+            const unsigned long long i = base + static_cast<unsigned>(j < sv ? j : sv - 1);
+            in[k] = op.load(i < nvec ? i : nvec - 1);
+        }
+#pragma unroll
+        for (int k = 0; k < NC; ++k) in[k].consume();
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const int j = threadIdx.x + k * T;
+            const unsigned long long i = base + static_cast<unsigned>(j < sv ? j : sv - 1);
+            const bool ok = j < sv && i < nvec;
+            const fvec<4> c = op.apply(i < nvec ? i : nvec - 1, in[k], bv[k], ok);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[k].v[e] += ok ? c.v[e] : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const int j = threadIdx.x + k * T;
+        if (j < sv) vstore<4>(lane_sums, j, acc[k]);
+    }
+    const int n = 4 * sv;
+    if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < tail) {
+        const Op1 op1 = op_from<Op1>(w0, w1, w2);
+        const size_t i = 4 * nvec + threadIdx.x;
+        const int c = cols - tail + static_cast<int>(threadIdx.x);
+        fvec<1> b = vzero<1>();
+        if (bias) b.v[0] = bias[c];
+        const typename Op1::In in = op1.load(i);
+        lane_sums[n + threadIdx.x] = op1.apply(i, in, b).v[0];
+    }
+    __syncthreads();
+    float* prow = part + static_cast<size_t>(blockIdx.x) * cols;
+    for (int c = threadIdx.x; c < cols; c += T) {
+        float s = lane_sums[c];
+        for (int x = c + cols; x < n; x += cols) s += lane_sums[x];
+        if (blockIdx.x == 0 && c >= cols - tail) s += lane_sums[n + c - (cols - tail)];
+        prow[c] = s;
+    }
+}
+
 template <int W>
 struct ResidBiasOp {  // out = (a + x) + bias
     const float* a;
@@ -762,6 +852,77 @@ int plan_reduce_parts(int rows, int nv) {
     return rows < MI_REDUCE_TILES ? rows : MI_REDUCE_TILES;
 }
 
+// Shape of the row-lane kernels: RL rows per workgroup and trip, NC vectors
+// per thread, T threads, `blocks` workgroups (partial rows).  rl == 0: not
+// for this shape.
+struct LanePlan {
+    int rl = 0, nc = 0, threads = 0, sv = 0, blocks = 0;
+};
+
+// Rows of at most 512 vectors take as many row lanes as fill 1024 threads
+// while the runs still go round kLaneBlocks workgroups; wider rows only where
+// their width is no multiple of 4 (one run of 4 or 2 rows, up to 4 vectors
+// per thread).  Rows of 513 to 4096 whole vectors stay with the row bands.
+// Below 16 columns the plain bands stay (a run must hold the tail elements'
+// columns, and such rows are never large).
+#ifndef MI_LANE_BLOCKS
+#define MI_LANE_BLOCKS 256
+#endif
+#ifndef MI_LANE_THREADS
+#define MI_LANE_THREADS 1024
+#endif
+constexpr int kLaneBlocks = MI_LANE_BLOCKS;
+constexpr int kLaneThreads = MI_LANE_THREADS;
+
+LanePlan plan_lanes(int rows, int cols) {
+    LanePlan p;
+    const int unit = cols % 4 == 0 ? 1 : cols % 2 == 0 ? 2 : 4;  // rows of a 16-byte aligned run
+    if (cols < 16 || cols > kMaxNC * 4096 / unit || (unit == 1 && cols > 2048)) return p;
+    const int sv1 = unit * cols / 4;
+    int m = kLaneThreads / sv1;  // units per run
+    const int most = rows / (unit * kLaneBlocks);
+    if (m > most) m = most;
+    if (m < 1) m = 1;
+    p.rl = m * unit;
+    p.sv = m * sv1;
+    p.nc = (p.sv + 1023) / 1024;
+    const int per = (p.sv + p.nc - 1) / p.nc;
+    p.threads = (per + kWave - 1) / kWave * kWave;
+    const long long runs = (static_cast<long long>(rows) + p.rl - 1) / p.rl;
+    p.blocks = static_cast<int>(runs < kLaneBlocks ? runs : kLaneBlocks);
+    return p;
+}
+
+template <class Op, class Op1>
+int launch_rowlane_reduce(const char* name, const LanePlan& p, Op op, const float* bias,
+                          float* dbias, int rows, int cols, hipStream_t st) {
+    int err = MI_OK;
+    char* ws = static_cast<char*>(workspace_get(colsum_bytes(p.blocks, cols), st, &err));
+    if (!ws) return err;
+    float* part = reinterpret_cast<float*>(ws + colsum_part_offset());
+    const unsigned long long total = static_cast<unsigned long long>(rows) * cols;
+    const OpWords ow = op_words(op);
+    const size_t lds = (4 * static_cast<size_t>(p.sv) + 4) * sizeof(float);
+#define MI_LANE_CASE(NN)                                                                       \
+    case NN:                                                                                   \
+        hipLaunchKernelGGL((rowlane_kernel<NN, Op, Op1>), dim3(p.blocks), dim3(p.threads), lds, \
+                           st, ow.w0, ow.w1, ow.w2, bias, total / 4, p.sv, p.threads, cols,    \
+                           p.blocks, static_cast<int>(total % 4), part);                       \
+        break;
+    switch (p.nc) {
+        MI_LANE_CASE(1)
+        MI_LANE_CASE(2)
+        MI_LANE_CASE(3)
+        MI_LANE_CASE(4)
+        default:
+            break;
+    }
+#undef MI_LANE_CASE
+    int rc = check_launch(name);
+    if (rc != MI_OK) return rc;
+    return launch_colsum_finalize(part, p.blocks, cols, dbias, cols, nullptr, st);
+}
+
 template <int W, class Op>
 int launch_rowtile_reduce(const char* name, Op op, const float* bias, float* dbias, int rows,
                           int cols, hipStream_t st) {
@@ -783,6 +944,23 @@ int launch_rowtile_reduce(const char* name, Op op, const float* bias, float* dbi
     int rc = check_launch(name);
     if (rc != MI_OK) return rc;
     return launch_colsum_finalize(part, P, cols, dbias, cols, nullptr, st);
+}
+
+// A reducing operator as its 16-byte form `op` and scalar form `op1` (the
+// same pointers); `aligned`: the tensors' own alignment allows 16-byte
+// accesses at every fourth element.
+template <class Op, class Op1>
+int launch_reduce(const char* name, Op op, Op1 op1, bool aligned, const float* bias, float* dbias,
+                  int rows, int cols, hipStream_t st) {
+    if (aligned) {
+        const LanePlan p = plan_lanes(rows, cols);
+        if (p.rl > 0)
+            return launch_rowlane_reduce<Op, Op1>(name, p, op, bias, dbias, rows, cols, st);
+        // 16-byte loads of the bias need its alignment too
+        if (cols % 4 == 0 && (!bias || aligned16(bias)))
+            return launch_rowtile_reduce<4>(name, op, bias, dbias, rows, cols, st);
+    }
+    return launch_rowtile_reduce<1>(name, op1, bias, dbias, rows, cols, st);
 }
 
 bool all_aligned(std::initializer_list<const void*> ps) {
@@ -889,11 +1067,8 @@ int mi_bias_backward(const float* grad, float* dbias, int rows, int cols, void* 
     if (int rc = check_shape(name, rows, cols)) return rc;
     if (rows == 0) return MI_OK;
     if (!grad || !dbias) return set_error(MI_ERR_INVALID_ARG, "%s: NULL", name);
-    if (cols % 4 == 0 && all_aligned({grad}))
-        return launch_rowtile_reduce<4>(name, ColSumOp<4>{grad}, nullptr, dbias, rows, cols,
-                                        to_stream(stream));
-    return launch_rowtile_reduce<1>(name, ColSumOp<1>{grad}, nullptr, dbias, rows, cols,
-                                    to_stream(stream));
+    return launch_reduce(name, ColSumOp<4>{grad}, ColSumOp<1>{grad}, all_aligned({grad}), nullptr,
+                         dbias, rows, cols, to_stream(stream));
 }
 
 int mi_relu_backward_with_bias_backward(const float* mask, const float* grad_out, float* grad_in,
@@ -903,11 +1078,10 @@ int mi_relu_backward_with_bias_backward(const float* mask, const float* grad_out
     if (rows == 0) return MI_OK;
     if (!mask || !grad_out || !grad_in || !dbias)
         return set_error(MI_ERR_INVALID_ARG, "%s: NULL", name);
-    if (cols % 4 == 0 && all_aligned({mask, grad_out, grad_in}))
-        return launch_rowtile_reduce<4>(name, ReluBwdBiasOp<4>{mask, grad_out, grad_in}, nullptr,
-                                        dbias, rows, cols, to_stream(stream));
-    return launch_rowtile_reduce<1>(name, ReluBwdBiasOp<1>{mask, grad_out, grad_in}, nullptr,
-                                    dbias, rows, cols, to_stream(stream));
+    return launch_reduce(name, ReluBwdBiasOp<4>{mask, grad_out, grad_in},
+                         ReluBwdBiasOp<1>{mask, grad_out, grad_in},
+                         all_aligned({mask, grad_out, grad_in}), nullptr, dbias, rows, cols,
+                         to_stream(stream));
 }
 
 int mi_gelu_backward_with_bias_backward(const float* in, const float* bias,
@@ -918,11 +1092,10 @@ int mi_gelu_backward_with_bias_backward(const float* in, const float* bias,
     if (rows == 0) return MI_OK;
     if (!in || !bias || !grad_out || !grad_in || !dbias)
         return set_error(MI_ERR_INVALID_ARG, "%s: NULL", name);
-    if (cols % 4 == 0 && all_aligned({in, bias, grad_out, grad_in}))
-        return launch_rowtile_reduce<4>(name, GeluBwdBiasOp<4>{in, grad_out, grad_in}, bias,
-                                        dbias, rows, cols, to_stream(stream));
-    return launch_rowtile_reduce<1>(name, GeluBwdBiasOp<1>{in, grad_out, grad_in}, bias, dbias,
-                                    rows, cols, to_stream(stream));
+    return launch_reduce(name, GeluBwdBiasOp<4>{in, grad_out, grad_in},
+                         GeluBwdBiasOp<1>{in, grad_out, grad_in},
+                         all_aligned({in, grad_out, grad_in}), bias, dbias, rows, cols,
+                         to_stream(stream));
 }
 
 }  // extern "C"
@@ -984,11 +1157,10 @@ int relu_bwd_mask16(const char* name, const void* mask, const float* grad_out, f
     if (!mask || !grad_out || !grad_in || !dbias)
         return set_error(MI_ERR_INVALID_ARG, "%s: NULL", name);
     const uint16_t* m = static_cast<const uint16_t*>(mask);
-    if (cols % 4 == 0 && aligned8(m) && all_aligned({grad_out, grad_in}))
-        return launch_rowtile_reduce<4>(name, ReluBwdMask16Op<4, T>{m, grad_out, grad_in},
-                                        nullptr, dbias, rows, cols, to_stream(stream));
-    return launch_rowtile_reduce<1>(name, ReluBwdMask16Op<1, T>{m, grad_out, grad_in}, nullptr,
-                                    dbias, rows, cols, to_stream(stream));
+    return launch_reduce(name, ReluBwdMask16Op<4, T>{m, grad_out, grad_in},
+                         ReluBwdMask16Op<1, T>{m, grad_out, grad_in},
+                         aligned8(m) && all_aligned({grad_out, grad_in}), nullptr, dbias, rows,
+                         cols, to_stream(stream));
 }
 
 }  // namespace

@@ -194,3 +194,56 @@ def test_gelu_unaligned_scalar_path(dev):
     Y = torch.zeros(rows * cols + 1, device=dev)[1:].view(rows, cols)
     M.bias_gelu_forward(X, dev_t(b), Y, rows, cols)
     assert_fwd("y", host(Y), O.bias_gelu_forward(x, b))
+
+
+def _offset(a, offset):
+    """On the GPU, `offset` elements into its allocation."""
+    flat = torch.from_numpy(np.ascontiguousarray(a)).reshape(-1)
+    buf = torch.empty(flat.numel() + offset, dtype=flat.dtype, device="cuda:0")
+    buf[offset:].copy_(flat)
+    return buf[offset:]
+
+
+# Row lanes: widths around their bounds (16 columns, 512 whole vectors, 4096
+# vectors of 2- and 4-row runs), row counts that leave a partial run, one to
+# three elements past the last vector, and tensors off 16 bytes.
+@pytest.mark.parametrize("rows,cols,off", [
+    (1, 15, 0), (1, 16, 0), (1, 17, 0), (3, 18, 0), (2, 19, 0), (255, 64, 0), (2049, 30, 0),
+    (1025, 511, 0), (1027, 512, 0), (2050, 127, 0), (513, 2048, 0), (513, 2052, 0), (300, 1025, 0),
+    (77, 2047, 0), (601, 4094, 0), (5, 4095, 0), (6, 4097, 0), (9, 8190, 0), (259, 8194, 0),
+    (1030, 96, 1), (7, 1002, 3),
+])
+def test_column_sums_row_lanes(dev, rows, cols, off):
+    note(f"row lanes rows={rows} cols={cols} off={off}")
+    x, b, g = gelu_inputs(rows, cols, rows + cols)
+    r = np.random.default_rng(cols)
+    db0 = r.standard_normal(cols, dtype=np.float32)
+    X, G, Bi = _offset(x, off), _offset(g, off), _offset(b, 1)
+    GIN = _offset(np.zeros_like(x), off)
+
+    DB = dev_t(db0)
+    M.bias_backward(G, DB, rows, cols)
+    assert_colsum("bias_backward", host(DB), O.bias_backward(g, db0), g)
+
+    gin_o, db_o = O.relu_backward_with_bias_backward(x, g, dbias=db0)
+    DB = dev_t(db0)
+    M.relu_backward_with_bias_backward(X, G, GIN, DB, rows, cols)
+    assert_exact("relu_bwd grad_in", host(GIN).reshape(rows, cols), gin_o)
+    assert_colsum("relu_bwd dbias", host(DB), db_o, gin_o)
+    again = dev_t(db0)
+    M.relu_backward_with_bias_backward(X, G, GIN, again, rows, cols)
+    assert_exact("relu_bwd dbias, again", host(again), host(DB))
+
+    h16 = x.astype(np.float16)
+    H = _offset(h16, off)
+    hin_o, hb_o = O.relu_backward_with_bias_backward_half_mask(h16.view(np.uint16), g, db0)
+    DB = dev_t(db0)
+    M.relu_backward_with_bias_backward_half_mask(H, G, GIN, DB, rows, cols)
+    assert_exact("half mask grad_in", host(GIN).reshape(rows, cols), hin_o)
+    assert_colsum("half mask dbias", host(DB), hb_o, hin_o)
+
+    gin64, db64 = O.gelu_backward_with_bias_backward_f64(x, b, g)
+    DB = dev_t(db0)
+    M.gelu_backward_with_bias_backward(X, Bi, G, GIN, DB, rows, cols)
+    assert_bwd("gelu grad_in", host(GIN).reshape(rows, cols), gin64)
+    assert_colsum("gelu dbias", host(DB), db64 + db0.astype(np.float64), gin64, approx_terms=True)
