@@ -178,6 +178,96 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     return t;
 }
 
+// Forward, a row over the G waves of a workgroup, held in registers: widths
+// past what one wave holds (4096 columns in 16-byte vectors, 1024 in scalars).
+// Memory-bound like the wave kernel; the block kernel below, which these
+// widths took before, walks the row three times in 4-byte accesses ([4096,
+// 5120] fwd + bwd 110 us, [3001, 1026] 23 us).  The statistics cost two LDS
+// exchanges.  gamma and beta of the next vector are requested before the
+// current one is stored: a load behind a store would wait for it (the
+// vector-memory counter retires in order).
+template <int W, int N, int G, bool SAVE, bool RESID>
+__global__ __launch_bounds__(G * kWave) void ln_fwd_group_kernel(
+    int rows, int cols, float eps, const float* __restrict__ a, const float* __restrict__ b,
+    const float* __restrict__ gamma, const float* __restrict__ beta, float* __restrict__ resid_out,
+    float* __restrict__ out, float* __restrict__ mean_out, float* __restrict__ rstd_out) {
+    constexpr int GT = G * kWave;
+    __shared__ float red[2][G];
+    const int row = blockIdx.x;
+    const int t = threadIdx.x;
+    const int wave = t / kWave;
+    const int nv = cols / W;
+    const size_t base = static_cast<size_t>(row) * cols;
+
+    fvec<W> v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int j = t + k * GT;
+        const int jj = j < nv ? j : nv - 1;
+        v[k] = sload<W>(a + base, jj);
+        if constexpr (RESID) {
+            const fvec<W> w = sload<W>(b + base, jj);
+#pragma unroll
+            for (int e = 0; e < W; ++e) v[k].v[e] = v[k].v[e] + w.v[e];
+        }
+    }
+    // Sum over the row's waves, in wave order; every thread gets it.
+    auto row_sum = [&](float x, int slot) __attribute__((always_inline)) {
+        const float w = wave_sum(x);
+        if ((t & (kWave - 1)) == 0) red[slot][wave] = w;
+        __syncthreads();
+        float r = red[slot][0];
+#pragma unroll
+        for (int i = 1; i < G; ++i) r += red[slot][i];
+        return r;
+    };
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const bool ok = t + k * GT < nv;
+#pragma unroll
+        for (int e = 0; e < W; ++e) s += ok ? v[k].v[e] : 0.0f;
+    }
+    const float mean = row_sum(s, 0) / static_cast<float>(cols);
+    float q = 0.0f;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const bool ok = t + k * GT < nv;
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+            const float d = ok ? v[k].v[e] - mean : 0.0f;
+            q += d * d;
+        }
+    }
+    const float var = row_sum(q, 1) / static_cast<float>(cols);
+    const float rstd = 1.0f / sqrtf(var + eps);
+
+    fvec<W> g = vload<W>(gamma, t < nv ? t : nv - 1);
+    fvec<W> bt = vload<W>(beta, t < nv ? t : nv - 1);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int j = t + k * GT;
+        fvec<W> y;
+#pragma unroll
+        for (int e = 0; e < W; ++e) y.v[e] = (v[k].v[e] - mean) * rstd * g.v[e] + bt.v[e];
+        if (k + 1 < N) {
+            const int jn = j + GT < nv ? j + GT : nv - 1;
+            g = vload<W>(gamma, jn);
+            bt = vload<W>(beta, jn);
+        }
+        if (j < nv) {
+            if constexpr (RESID) sstore<W>(resid_out + base, j, v[k]);
+            sstore<W>(out + base, j, y);
+        }
+    }
+    if constexpr (SAVE) {
+        if (t == 0) {
+            mean_out[row] = mean;
+            rstd_out[row] = rstd;
+        }
+    }
+}
+
 // Forward, one block per row, any width (streams the row three times).
 template <bool SAVE, bool RESID>
 __global__ __launch_bounds__(kBlockThreads) void ln_fwd_block_kernel(
@@ -403,7 +493,7 @@ __global__ __launch_bounds__(NWV * kWave) void ln_bwd_group_kernel(
     // 1600]: 34.0 against 36.7 us; [32768, 1600]: 109.0 against 124.1 us);
     // with 4 vectors per lane the second row costs occupancy ([32768, 4096]:
     // 290 against 269 us).
-    constexpr int RF = (G > 1 && N <= 2) ? 2 : 1;
+    constexpr int RF = (G > 1 && N * W <= 8) ? 2 : 1;
     const int first = blockIdx.x * GPB;
     const unsigned iters = strided_trips(static_cast<unsigned>(first), static_cast<unsigned>(rows),
                                          static_cast<unsigned>(stride));
@@ -549,8 +639,163 @@ __global__ __launch_bounds__(kBlockThreads) void ln_bwd_block_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// Narrow rows (at most 32 16-byte vectors): L = 16 or 32 lanes own a row, one
+// vector per lane, so a wave holds 4 or 2 rows.  With a whole wave per row,
+// half of its lanes or more had no work and each wave kept one short row in
+// flight ([65536, 96] fwd + bwd 48 us).
+// ---------------------------------------------------------------------------
+
+// Sum over the L lanes of a row, in every one of them; fixed order.
+template <int L>
+__device__ __forceinline__ float sub_sum(float v) {
+    v += dpp_move<0xB1>(v);
+    v += dpp_move<0x4E>(v);
+    v += dpp_move<0x141>(v);
+    v += dpp_move<0x140>(v);
+    if constexpr (L == 32) v += __shfl_xor(v, 16, kWave);
+    return v;
+}
+
+template <int L, bool SAVE, bool RESID>
+__global__ __launch_bounds__(kBlockThreads) void ln_fwd_sub_kernel(
+    int rows, int cols, float eps, const float* __restrict__ a, const float* __restrict__ b,
+    const float* __restrict__ gamma, const float* __restrict__ beta, float* __restrict__ resid_out,
+    float* __restrict__ out, float* __restrict__ mean_out, float* __restrict__ rstd_out) {
+    const int j = threadIdx.x % L;
+    const int row = blockIdx.x * (kBlockThreads / L) + static_cast<int>(threadIdx.x) / L;
+    const int nv = cols / 4;
+    const bool ok = row < rows && j < nv;
+    const int jj = j < nv ? j : nv - 1;
+    const size_t base = static_cast<size_t>(row < rows ? row : rows - 1) * cols;
+    fvec<4> v = sload<4>(a + base, jj);
+    if constexpr (RESID) {
+        const fvec<4> w = sload<4>(b + base, jj);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v.v[e] = v.v[e] + w.v[e];
+    }
+    const fvec<4> g = vload<4>(gamma, jj);
+    const fvec<4> bt = vload<4>(beta, jj);
+    float s = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s += j < nv ? v.v[e] : 0.0f;
+    const float mean = sub_sum<L>(s) / static_cast<float>(cols);
+    float q = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float d = j < nv ? v.v[e] - mean : 0.0f;
+        q += d * d;
+    }
+    const float var = sub_sum<L>(q) / static_cast<float>(cols);
+    const float rstd = 1.0f / sqrtf(var + eps);
+    if (ok) {
+        fvec<4> y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y.v[e] = (v.v[e] - mean) * rstd * g.v[e] + bt.v[e];
+        if constexpr (RESID) sstore<4>(resid_out + base, j, v);
+        sstore<4>(out + base, j, y);
+        if constexpr (SAVE) {
+            if (j == 0) {
+                mean_out[row] = mean;
+                rstd_out[row] = rstd;
+            }
+        }
+    }
+}
+
+// Backward, T threads per workgroup (T / L rows at a time), RF rows per lane
+// group in flight; the groups' sums are staged in LDS as [2 * cols] rows and
+// added in group order into the workgroup's partial row.
+constexpr int kSubRows = 2;
+
+template <int L, bool ADD>
+__global__ __launch_bounds__(1024) void ln_bwd_sub_kernel(
+    int rows, int cols, int nblk, int T, const float* __restrict__ gout,
+    const float* __restrict__ x, const float* __restrict__ gamma, float* __restrict__ gx,
+    const float* __restrict__ mean, const float* __restrict__ rstd, float* __restrict__ part) {
+    extern __shared__ __align__(16) float sub_sums[];
+    const int j = threadIdx.x % L;
+    const int grp = static_cast<int>(threadIdx.x) / L;
+    const int gpb = T / L;
+    const int nv = cols / 4;
+    const int jj = j < nv ? j : nv - 1;
+    fvec<4> gm = vload<4>(gamma, jj);
+    fvec<4> ag = vzero<4>(), ab = vzero<4>();
+    const unsigned stride = static_cast<unsigned>(nblk * gpb);
+    for (unsigned r0 = blockIdx.x * static_cast<unsigned>(gpb) + static_cast<unsigned>(grp);
+         r0 - static_cast<unsigned>(grp) < static_cast<unsigned>(rows); r0 += kSubRows * stride) {
+        // The trip count is uniform over the workgroup; rows past the end
+        // load the last row and add zeros.
+        fvec<4> go[kSubRows], xv[kSubRows], old[kSubRows];
+        float mu[kSubRows], is[kSubRows];
+        size_t off[kSubRows];
+        bool ok[kSubRows];
+#pragma unroll
+        for (int r = 0; r < kSubRows; ++r) {
+            const unsigned row = r0 + static_cast<unsigned>(r) * stride;
+            const unsigned rr = row < static_cast<unsigned>(rows) ? row : static_cast<unsigned>(rows) - 1u;
+            ok[r] = row < static_cast<unsigned>(rows) && j < nv;
+            off[r] = static_cast<size_t>(rr) * cols;
+            go[r] = sload<4>(gout + off[r], jj);
+            xv[r] = sload<4>(x + off[r], jj);
+            if constexpr (ADD) old[r] = sload<4>(gx + off[r], jj);
+            mu[r] = mean[rr];
+            is[r] = rstd[rr];
+        }
+#pragma unroll
+        for (int r = 0; r < kSubRows; ++r) {
+            float s1 = 0.0f, s2 = 0.0f;
+            fvec<4> xh, g;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                g.v[e] = ok[r] ? go[r].v[e] : 0.0f;
+                xh.v[e] = (xv[r].v[e] - mu[r]) * is[r];
+                const float dh = g.v[e] * gm.v[e];
+                s1 += dh;
+                s2 += dh * xh.v[e];
+                ag.v[e] += g.v[e] * xh.v[e];
+                ab.v[e] += g.v[e];
+            }
+            const float m1 = sub_sum<L>(s1) / static_cast<float>(cols);
+            const float m2 = sub_sum<L>(s2) / static_cast<float>(cols);
+            if constexpr (ADD) consume(old[r]);
+            if (ok[r]) {
+                fvec<4> d;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float dh = g.v[e] * gm.v[e];
+                    const float dx = is[r] * (dh - m1 - xh.v[e] * m2);
+                    if constexpr (ADD)
+                        d.v[e] = old[r].v[e] + rounded(dx);
+                    else
+                        d.v[e] = dx;
+                }
+                sstore<4>(gx + off[r], j, d);
+            }
+        }
+    }
+    float* mine = sub_sums + static_cast<size_t>(grp) * 2 * cols;
+    if (j < nv) {
+        vstore<4>(mine, j, ag);
+        vstore<4>(mine + cols, j, ab);
+    }
+    __syncthreads();
+    float* prow = part + static_cast<size_t>(blockIdx.x) * 2 * cols;
+    for (int c = threadIdx.x; c < 2 * cols; c += T) {
+        float t = sub_sums[c];
+        for (int i = 1; i < gpb; ++i) t += sub_sums[i * 2 * cols + c];
+        prow[c] = t;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Host dispatch.
 // ---------------------------------------------------------------------------
+
+// Lanes per row of the narrow-row kernels, 0 where a wave per row is used.
+int sub_lanes(int cols, bool vec4) {
+    if (!vec4 || cols > 128) return 0;
+    return cols <= 64 ? 16 : 32;
+}
 
 // Smallest supported vectors-per-lane count >= need, or 0 if none.
 int pick_n(int need) {
@@ -603,6 +848,48 @@ void launch_fwd_wave(int n, hipStream_t st, const float* a, const float* b, cons
 #undef MI_LN_FWD_CASE
 }
 
+// Rows over G waves: G and the vectors per lane for rows of nv vectors (more
+// than one wave holds), or 0 beyond 16 waves of 12 vectors (16 would spill).
+struct FwdGroup {
+    int g = 0, n = 0;
+};
+
+FwdGroup fwd_group(int nv) {
+    static const int kN[] = {5, 6, 8, 10, 12, 16};
+    for (int g = 4; g <= 16; g *= 4)
+        for (int n : kN)
+            if (n * g * kWave >= nv && (g == 4 || n <= 12)) return {g, n};
+    return {};
+}
+
+template <int W, int G, bool SAVE, bool RESID>
+void launch_fwd_group(int n, hipStream_t st, const float* a, const float* b, const float* gamma,
+                      const float* beta, float* ro, float* out, float* mo, float* so, int rows,
+                      int cols, float eps) {
+#define MI_LN_FWD_CASE(NN)                                                                      \
+    case NN:                                                                                    \
+        hipLaunchKernelGGL((ln_fwd_group_kernel<W, NN, G, SAVE, RESID>), dim3(rows),            \
+                           dim3(G * kWave), 0, st, rows, cols, eps, a, b, gamma, beta, ro, out, \
+                           mo, so);                                                             \
+        break;
+    switch (n) {
+        MI_LN_FWD_CASE(5)
+        MI_LN_FWD_CASE(6)
+        MI_LN_FWD_CASE(8)
+        MI_LN_FWD_CASE(10)
+        MI_LN_FWD_CASE(12)
+        default:
+            if constexpr (G == 4) {
+                switch (n) {
+                    MI_LN_FWD_CASE(16)
+                    default: break;
+                }
+            }
+            break;
+    }
+#undef MI_LN_FWD_CASE
+}
+
 template <bool SAVE, bool RESID>
 int ln_forward_impl(const char* name, const float* a, const float* b, const float* gamma,
                     const float* beta, float* ro, float* out, float* mo, float* so, int rows,
@@ -615,6 +902,17 @@ int ln_forward_impl(const char* name, const float* a, const float* b, const floa
         return set_error(MI_ERR_INVALID_ARG, "%s: NULL pointer", name);
     const bool vec4 = (cols % 4 == 0) && aligned16(a) && aligned16(gamma) && aligned16(beta) &&
                       aligned16(out) && (!RESID || (aligned16(b) && aligned16(ro)));
+    if (const int lanes = sub_lanes(cols, vec4)) {
+        const int per = kBlockThreads / lanes;  // rows per workgroup
+        const dim3 grid(static_cast<unsigned>((static_cast<long long>(rows) + per - 1) / per));
+        if (lanes == 16)
+            hipLaunchKernelGGL((ln_fwd_sub_kernel<16, SAVE, RESID>), grid, dim3(kBlockThreads), 0,
+                               st, rows, cols, eps, a, b, gamma, beta, ro, out, mo, so);
+        else
+            hipLaunchKernelGGL((ln_fwd_sub_kernel<32, SAVE, RESID>), grid, dim3(kBlockThreads), 0,
+                               st, rows, cols, eps, a, b, gamma, beta, ro, out, mo, so);
+        return check_launch(name);
+    }
     const int W = vec4 ? 4 : 1;
     const int need = (cols / W + kWave - 1) / kWave;
     const int n = pick_n(need);
@@ -632,6 +930,19 @@ int ln_forward_impl(const char* name, const float* a, const float* b, const floa
         else
             launch_fwd_wave<1, 1, SAVE, RESID>(n, st, a, b, gamma, beta, ro, out, mo, so, rows,
                                                cols, eps);
+    } else if (const FwdGroup fg = fwd_group(cols / W); fg.g != 0) {
+        if (vec4 && fg.g == 4)
+            launch_fwd_group<4, 4, SAVE, RESID>(fg.n, st, a, b, gamma, beta, ro, out, mo, so, rows,
+                                                cols, eps);
+        else if (vec4)
+            launch_fwd_group<4, 16, SAVE, RESID>(fg.n, st, a, b, gamma, beta, ro, out, mo, so,
+                                                 rows, cols, eps);
+        else if (fg.g == 4)
+            launch_fwd_group<1, 4, SAVE, RESID>(fg.n, st, a, b, gamma, beta, ro, out, mo, so, rows,
+                                                cols, eps);
+        else
+            launch_fwd_group<1, 16, SAVE, RESID>(fg.n, st, a, b, gamma, beta, ro, out, mo, so,
+                                                 rows, cols, eps);
     } else {
         hipLaunchKernelGGL((ln_fwd_block_kernel<SAVE, RESID>), dim3(rows), dim3(kBlockThreads), 0,
                            st, rows, cols, eps, a, b, gamma, beta, ro, out, mo, so);
@@ -641,6 +952,7 @@ int ln_forward_impl(const char* name, const float* a, const float* b, const floa
 
 struct BwdPlan {
     int W = 1, N = 0, G = 1;  // N == 0: block-per-row fallback
+    int lanes = 0;            // > 0: the narrow-row kernels, `waves` waves
     int waves = kBwdWaves;    // waves per workgroup
     int blocks = 0;
     size_t lds = 0;
@@ -650,18 +962,36 @@ BwdPlan plan_bwd(int rows, int cols, bool vec4, bool add) {
     BwdPlan p;
     p.W = vec4 ? 4 : 1;
     const int nv = cols / p.W;
-    // N <= 6 keeps the combine LDS at or under 48 KB (G = 1: 4 slots of
-    // 2*N*W*64 floats; G = 4: 1 slot of 2*N*W*256 floats; G = 8: one group
-    // per workgroup, no combine) and the registers within budget (N = 8 with
-    // W = 4 spills).  Wider rows use the block-per-row kernel.
+    p.lanes = sub_lanes(cols, vec4);
+    if (p.lanes) {
+        // As many rows per workgroup as keep MI_LN_BWD_MAX_BLOCKS workgroups
+        // busy, 4 to 16 waves.
+        p.waves = 16;
+        while (p.waves > 4 && static_cast<long long>(p.waves) * kWave / p.lanes *
+                                      MI_LN_BWD_MAX_BLOCKS > rows)
+            p.waves /= 2;
+        const int gpb = p.waves * kWave / p.lanes;
+        const long long groups = (static_cast<long long>(rows) + gpb - 1) / gpb;
+        p.blocks = static_cast<int>(groups < MI_LN_BWD_MAX_BLOCKS ? groups : MI_LN_BWD_MAX_BLOCKS);
+        if (p.blocks < 1) p.blocks = 1;
+        p.lds = static_cast<size_t>(gpb) * 2 * cols * sizeof(float);
+        return p;
+    }
+    // 16-byte vectors: N <= 6 keeps the combine LDS at or under 48 KB (G = 1:
+    // 4 slots of 2*N*W*64 floats; G = 4: 1 slot of 2*N*W*256 floats; one group
+    // per workgroup beyond: no combine) and the registers within budget
+    // (N = 8 spills).  Scalars hold four times fewer floats per vector, so
+    // N goes to 16, which keeps a row on as few waves (with N <= 6, 8 waves
+    // of 2 to 6 floats per lane and a barrier per row: [16384, 999] fwd + bwd
+    // 81 us).  Wider rows use the block-per-row kernel.
     static const int kG[] = {1, 4, 8};
-    static const int kMaxN[] = {6, 6, 6};
-    static const int kN[] = {1, 2, 3, 4, 6};
+    static const int kN[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    const int max_n = p.W == 4 ? 6 : 16;
     for (int gi = 0; gi < 3 && !p.N; ++gi) {
         const int g = kG[gi];
         const int need = (nv + g * kWave - 1) / (g * kWave);
         for (int n : kN)
-            if (n >= need && n <= kMaxN[gi]) {
+            if (n >= need && n <= max_n) {
                 p.N = n;
                 p.G = g;
                 break;
@@ -679,7 +1009,7 @@ BwdPlan plan_bwd(int rows, int cols, bool vec4, bool add) {
         // twice the waves per CU pay off (GPT-2-small block x12 2011.6 ->
         // 1988.1 us; GPT-2-XL-shaped block x48 8.80 -> 8.55 ms), where the
         // plain form is 0.7 us slower that way at [8192, 768].
-        p.waves = (p.G == 4 && p.N == 4)                ? 4
+        p.waves = (p.W == 4 && p.G == 4 && p.N == 4) ? 4
                   : (add && ((p.G == 1 && p.N <= 3) || (p.G == 4 && p.N <= 2))) ? 16
                                                          : kBwdWaves;
         const int maxb = p.waves == 4 ? 2 * MI_LN_BWD_MAX_BLOCKS : MI_LN_BWD_MAX_BLOCKS;
@@ -708,7 +1038,7 @@ void launch_bwd_group(const BwdPlan& p, hipStream_t st, const float* g, const fl
             return;
         }
     }
-    if constexpr (G == 4 && N == 4) {
+    if constexpr (W == 4 && G == 4 && N == 4) {
         if (p.waves == 4) {
             hipLaunchKernelGGL((ln_bwd_group_kernel<W, N, G, ADD, 4>), dim3(p.blocks),
                                dim3(4 * kWave), p.lds, st, rows, cols, p.blocks, g, x, gamma,
@@ -732,6 +1062,14 @@ void dispatch_bwd_n(const BwdPlan& p, hipStream_t st, const float* g, const floa
         case 4: launch_bwd_group<W, 4, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
         case 6: launch_bwd_group<W, 6, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
         default: break;
+    }
+    if constexpr (W == 1) {
+        switch (p.N) {
+            case 8: launch_bwd_group<W, 8, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
+            case 12: launch_bwd_group<W, 12, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
+            case 16: launch_bwd_group<W, 16, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
+            default: break;
+        }
     }
 }
 
@@ -779,7 +1117,15 @@ int ln_backward_launch(const char* name, const BwdPlan& p, const float* g, const
                        const float* m, const float* s, const float* gamma, float* gx,
                        float* dgamma, float* dbeta, float* part, int rows, int cols,
                        hipStream_t st) {
-    if (p.N) {
+    if (p.lanes) {
+        const dim3 grid(p.blocks), block(p.waves * kWave);
+        if (p.lanes == 16)
+            hipLaunchKernelGGL((ln_bwd_sub_kernel<16, ADD>), grid, block, p.lds, st, rows, cols,
+                               p.blocks, p.waves * kWave, g, x, gamma, gx, m, s, part);
+        else
+            hipLaunchKernelGGL((ln_bwd_sub_kernel<32, ADD>), grid, block, p.lds, st, rows, cols,
+                               p.blocks, p.waves * kWave, g, x, gamma, gx, m, s, part);
+    } else if (p.N) {
         if (p.W == 4)
             dispatch_bwd_g<4, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols);
         else
