@@ -46,7 +46,20 @@ constexpr int sm_threads() {
     return (G < 4 ? 4 : G) * kWave;
 }
 
-template <int G, int K, bool CE>
+// V = 4 takes 16-byte accesses (cols % 4 == 0 and 16-byte aligned tensors), V
+// = 1 4-byte ones; K accesses per lane.
+//
+// Memory-bound.  16-byte stores carry the non-temporal hint, and rows over 8
+// waves or more (past 2048 columns) load with it too; [16384, 1024] softmax 34.8 -> 21.0
+// us (28.7 without the hint, 24.8 with it on the loads too), [16384, 1100]
+// 51.5 -> 23.1, [4096, 32000] 195 -> 176 (181 with stores alone), cross-entropy
+// [8192, 32000] 374 -> 348.  4-byte accesses do better without: their rows
+// start anywhere, and lines shared by two waves are then written twice.
+// Sharing one long row between workgroups that each read all of it and store
+// a part was slower ([64, 32000] 7.1 -> 8.8 us, 16 rows of 50257 9.4 -> 21).
+constexpr int kNontemporal = 2;  // cache-policy bit of the buffer accesses
+
+template <int G, int K, bool CE, int V>
 __global__ __launch_bounds__(sm_threads<G>()) void row_softmax_kernel(
     const float* __restrict__ x, float* __restrict__ out, int rows, int cols,
     const int* __restrict__ targets, float* __restrict__ losses, float scale) {
@@ -68,19 +81,29 @@ __global__ __launch_bounds__(sm_threads<G>()) void row_softmax_kernel(
 
     // Raw buffer loads bounded by the row length: slots past the end read 0
     // in hardware, so no index is clamped and every load shares one lane
-    // offset (t * 4) plus a per-slot scalar offset.  Masked slots then take
+    // offset plus a per-slot scalar offset.  Masked slots then take
     // -FLT_MAX, the reference's initial maximum, and give exp(.) = 0 below.
     const __amdgpu_buffer_rsrc_t rin = row_rsrc(xr, cols);
-    float v[K];
+    float v[K][V];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const float a = __int_as_float(
-            __builtin_amdgcn_raw_buffer_load_b32(rin, t * 4, k * GT * 4, 0));
-        v[k] = (t + k * GT) < cols ? a : -FLT_MAX;
+        if constexpr (V == 4) {
+            const auto a = __builtin_amdgcn_raw_buffer_load_b128(rin, t * 16, k * GT * 16,
+                                                                 G >= 8 ? kNontemporal : 0);
+            const bool ok = 4 * (t + k * GT) < cols;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[k][e] = ok ? __int_as_float(a[e]) : -FLT_MAX;
+        } else {
+            const float a =
+                __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rin, t * 4, k * GT * 4, 0));
+            v[k][0] = (t + k * GT) < cols ? a : -FLT_MAX;
+        }
     }
     float m = -FLT_MAX;
 #pragma unroll
-    for (int k = 0; k < K; ++k) m = fmaxf(m, v[k]);
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int e = 0; e < V; ++e) m = fmaxf(m, v[k][e]);
     m = wave_max(m);
     if constexpr (G > 1) {
         if (lane == 0) red_max[grp][wig] = m;
@@ -97,11 +120,13 @@ __global__ __launch_bounds__(sm_threads<G>()) void row_softmax_kernel(
     const float mL = m * kLog2e;
     float s = 0.0f;
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(v[k], kLog2e, -mL));
-        v[k] = e;
-        s += e;
-    }
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const float ex = __builtin_amdgcn_exp2f(fmaf(v[k][e], kLog2e, -mL));
+            v[k][e] = ex;
+            s += ex;
+        }
     s = wave_sum(s);
     if constexpr (G > 1) {
         if (lane == 0) red_sum[grp][wig] = s;
@@ -114,28 +139,50 @@ __global__ __launch_bounds__(sm_threads<G>()) void row_softmax_kernel(
 
     // Buffer stores past the row end are dropped in hardware.
     const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + static_cast<size_t>(row) * cols, cols);
+    auto store = [&](int k, const float (&y)[V]) __attribute__((always_inline)) {
+        if constexpr (V == 4) {
+            typedef int i32x4 __attribute__((ext_vector_type(4)));
+            const i32x4 q = {__float_as_int(y[0]), __float_as_int(y[1]), __float_as_int(y[2]),
+                             __float_as_int(y[3])};
+            // The slot's offset is in the lane offset, not a scalar one: a
+            // 16-byte buffer store must not be followed at once by a write of
+            // its data registers, and the compiler leaves that wait out for
+            // stores with a scalar offset register, which gave wrong first
+            // elements here.
+            __builtin_amdgcn_raw_buffer_store_b128(q, rout, (t + k * GT) * 16, 0, kNontemporal);
+        } else {
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(y[0]), rout, t * 4, k * GT * 4, 0);
+        }
+    };
     if constexpr (!CE) {
         const float inv = 1.0f / s;
 #pragma unroll
-        for (int k = 0; k < K; ++k)
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v[k] * inv), rout, t * 4,
-                                                  k * GT * 4, 0);
+        for (int k = 0; k < K; ++k) {
+            float y[V];
+#pragma unroll
+            for (int e = 0; e < V; ++e) y[e] = v[k][e] * inv;
+            store(k, y);
+        }
     } else {
         const float inv = 1.0f / (s + kCeEps);
         const int tgt = targets[row];
         float pt = 0.0f;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            const float p = v[k] * inv;
-            const bool hit = (t + k * GT) == tgt;
-            pt = hit ? p : pt;
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_int((hit ? p - 1.0f : p) * scale),
-                                                  rout, t * 4, k * GT * 4, 0);
+            float y[V];
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                const float p = v[k][e] * inv;
+                const bool hit = V * (t + k * GT) + e == tgt;
+                pt = hit ? p : pt;
+                y[e] = (hit ? p - 1.0f : p) * scale;
+            }
+            store(k, y);
         }
         // One lane owns the target and writes the loss; an invalid target
         // gives NaN (written by lane 0 of the group).
         if (tgt >= 0 && tgt < cols) {
-            if (tgt % GT == t) losses[row] = -logf(pt + kCeEps);
+            if (tgt / V % GT == t) losses[row] = -logf(pt + kCeEps);
         } else if (t == 0) {
             losses[row] = __int_as_float(0x7fc00000);
         }
@@ -214,54 +261,97 @@ struct SmPlan {
     int G = 0, K = 0;  // G == 0: long-row kernel
 };
 
-SmPlan plan_softmax(int cols) {
-    const int slots = (cols + kWave - 1) / kWave;  // lane slots for one wave
-    if (slots <= 16) {
-        int k = 1;
-        while (k < slots) k *= 2;
-        return {1, k};
+// The fewest waves, then the fewest accesses per lane that hold the row.  An
+// access is 16 bytes (vec4) or 4.
+SmPlan plan_softmax(int cols, bool vec4) {
+    static const int kK1[] = {1, 2, 3, 4, 6, 8, 10, 12, 14, 16};
+    static const int kK16[] = {10, 12, 14, 16, 24, 32, 40, 48, 56, 64};
+    static const int kV1[] = {1, 2, 3, 4};
+    static const int kV16[] = {3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
+    const int n = vec4 ? cols / 4 : cols;  // accesses
+    for (int g = 1; g <= 16; g *= 2) {
+        if (vec4 && g < 16) {
+            for (int k : kV1)
+                if (n <= g * kWave * k) return {g, k};
+        } else {
+            for (int k : (g < 16 ? kK1 : vec4 ? kV16 : kK16))
+                if (n <= g * kWave * k) return {g, k};
+        }
     }
-    if (cols <= 2 * kWave * 16) return {2, 16};
-    if (cols <= 4 * kWave * 16) return {4, 16};
-    if (cols <= 8 * kWave * 16) return {8, 16};
-    for (int k = 16; k <= 64; k += 8)
-        if (cols <= 16 * kWave * k) return {16, k};
     return {};
 }
 
-template <int G, int K, bool CE>
+template <int G, int K, bool CE, int V>
 void launch_rows(int rows, int cols, hipStream_t st, const float* x, float* out, const int* tg,
                  float* losses, float scale) {
     constexpr int GPB = G < 4 ? 4 / G : 1;
     const dim3 grid(static_cast<unsigned>((static_cast<long long>(rows) + GPB - 1) / GPB));
-    hipLaunchKernelGGL((row_softmax_kernel<G, K, CE>), grid, dim3(sm_threads<G>()), 0, st, x, out,
-                       rows, cols, tg, losses, scale);
+    hipLaunchKernelGGL((row_softmax_kernel<G, K, CE, V>), grid, dim3(sm_threads<G>()), 0, st, x,
+                       out, rows, cols, tg, losses, scale);
 }
 
 template <bool CE>
 void launch_softmax(int rows, int cols, hipStream_t st, const float* x, float* out, const int* tg,
                     float* losses, float scale) {
-    const SmPlan p = plan_softmax(cols);
-#define MI_SM_CASE(GG, KK)                                                       \
-    if (p.G == GG && p.K == KK) {                                                \
-        launch_rows<GG, KK, CE>(rows, cols, st, x, out, tg, losses, scale);      \
+    const bool vec4 = cols % 4 == 0 && aligned16(x) && aligned16(out);
+    const SmPlan p = plan_softmax(cols, vec4);
+#define MI_SM_CASE(GG, KK, VV)                                                  \
+    if (p.G == GG && p.K == KK && vec4 == (VV == 4)) {                           \
+        launch_rows<GG, KK, CE, VV>(rows, cols, st, x, out, tg, losses, scale);  \
         return;                                                                  \
     }
-    MI_SM_CASE(1, 1)
-    MI_SM_CASE(1, 2)
-    MI_SM_CASE(1, 4)
-    MI_SM_CASE(1, 8)
-    MI_SM_CASE(1, 16)
-    MI_SM_CASE(2, 16)
-    MI_SM_CASE(4, 16)
-    MI_SM_CASE(8, 16)
-    MI_SM_CASE(16, 16)
-    MI_SM_CASE(16, 24)
-    MI_SM_CASE(16, 32)
-    MI_SM_CASE(16, 40)
-    MI_SM_CASE(16, 48)
-    MI_SM_CASE(16, 56)
-    MI_SM_CASE(16, 64)
+    MI_SM_CASE(1, 1, 4)
+    MI_SM_CASE(1, 2, 4)
+    MI_SM_CASE(1, 3, 4)
+    MI_SM_CASE(1, 4, 4)
+    MI_SM_CASE(2, 3, 4)
+    MI_SM_CASE(2, 4, 4)
+    MI_SM_CASE(4, 3, 4)
+    MI_SM_CASE(4, 4, 4)
+    MI_SM_CASE(8, 3, 4)
+    MI_SM_CASE(8, 4, 4)
+    MI_SM_CASE(16, 3, 4)
+    MI_SM_CASE(16, 4, 4)
+    MI_SM_CASE(16, 5, 4)
+    MI_SM_CASE(16, 6, 4)
+    MI_SM_CASE(16, 7, 4)
+    MI_SM_CASE(16, 8, 4)
+    MI_SM_CASE(16, 10, 4)
+    MI_SM_CASE(16, 12, 4)
+    MI_SM_CASE(16, 14, 4)
+    MI_SM_CASE(16, 16, 4)
+    MI_SM_CASE(1, 1, 1)
+    MI_SM_CASE(1, 2, 1)
+    MI_SM_CASE(1, 3, 1)
+    MI_SM_CASE(1, 4, 1)
+    MI_SM_CASE(1, 6, 1)
+    MI_SM_CASE(1, 8, 1)
+    MI_SM_CASE(1, 10, 1)
+    MI_SM_CASE(1, 12, 1)
+    MI_SM_CASE(1, 14, 1)
+    MI_SM_CASE(1, 16, 1)
+    MI_SM_CASE(2, 10, 1)
+    MI_SM_CASE(2, 12, 1)
+    MI_SM_CASE(2, 14, 1)
+    MI_SM_CASE(2, 16, 1)
+    MI_SM_CASE(4, 10, 1)
+    MI_SM_CASE(4, 12, 1)
+    MI_SM_CASE(4, 14, 1)
+    MI_SM_CASE(4, 16, 1)
+    MI_SM_CASE(8, 10, 1)
+    MI_SM_CASE(8, 12, 1)
+    MI_SM_CASE(8, 14, 1)
+    MI_SM_CASE(8, 16, 1)
+    MI_SM_CASE(16, 10, 1)
+    MI_SM_CASE(16, 12, 1)
+    MI_SM_CASE(16, 14, 1)
+    MI_SM_CASE(16, 16, 1)
+    MI_SM_CASE(16, 24, 1)
+    MI_SM_CASE(16, 32, 1)
+    MI_SM_CASE(16, 40, 1)
+    MI_SM_CASE(16, 48, 1)
+    MI_SM_CASE(16, 56, 1)
+    MI_SM_CASE(16, 64, 1)
 #undef MI_SM_CASE
     hipLaunchKernelGGL((long_row_softmax_kernel<CE>), dim3(rows), dim3(kLongThreads), 0, st, x,
                        out, cols, tg, losses, scale);

@@ -152,3 +152,29 @@ def test_model_size_cross_entropy(dev):
     assert_fwd("losses", host(losses), lr)
     assert_bwd("grad", host(G), gr)
     assert_fwd("mean loss", host(lout)[0], np.float32(O.loss_mean(lr)))
+
+
+# Edges of the row shapes: accesses per lane and waves per row, with 16-byte
+# accesses (widths of whole vectors) and 4-byte ones, the longest register
+# rows and the first past them.
+@pytest.mark.parametrize("rows,cols", [
+    (5, 252), (9, 256), (3, 260), (7, 1020), (5, 1028), (3, 1540), (3, 2052), (2, 4100),
+    (2, 8196), (3, 12292), (2, 28676), (1, 65532), (1, 65540),
+    (5, 385), (6, 641), (3, 1025), (3, 1281), (2, 2561), (3, 5121), (2, 9217), (1, 40961),
+])
+def test_row_shape_edges(dev, rows, cols):
+    test_softmax_shapes(dev, rows, cols)
+    test_cross_entropy_shapes_v1_and_v2(dev, rows, cols)
+
+
+def test_unaligned_rows_take_the_scalar_accesses(dev):
+    rows, cols = 5, 1024
+    x, _ = _logits(rows, cols, 3)
+    X = torch.zeros(rows * cols + 1, device="cuda")[1:]
+    X.copy_(dev_t(x).reshape(-1))
+    Y = torch.empty(rows, cols, device="cuda")
+    M.softmax_forward(X, Y, rows, cols)
+    assert_fwd("softmax, unaligned", host(Y), O.softmax_forward_f64(x))
+    Z = dev_t(x)
+    M.softmax_forward(Z, Z, rows, cols)   # in place
+    assert_fwd("softmax, in place", host(Z), O.softmax_forward_f64(x))
