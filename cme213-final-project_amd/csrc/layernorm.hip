@@ -848,6 +848,8 @@ void launch_fwd_wave(int n, hipStream_t st, const float* a, const float* b, cons
 #undef MI_LN_FWD_CASE
 }
 
+constexpr int kFewRows = 1024;
+
 // Rows over G waves: G and the vectors per lane for rows of nv vectors (more
 // than one wave holds), or 0 beyond 16 waves of 12 vectors (16 would spill).
 struct FwdGroup {
@@ -855,7 +857,7 @@ struct FwdGroup {
 };
 
 FwdGroup fwd_group(int nv) {
-    static const int kN[] = {5, 6, 8, 10, 12, 16};
+    static const int kN[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
     for (int g = 4; g <= 16; g *= 4)
         for (int n : kN)
             if (n * g * kWave >= nv && (g == 4 || n <= 12)) return {g, n};
@@ -881,6 +883,10 @@ void launch_fwd_group(int n, hipStream_t st, const float* a, const float* b, con
         default:
             if constexpr (G == 4) {
                 switch (n) {
+                    MI_LN_FWD_CASE(1)
+                    MI_LN_FWD_CASE(2)
+                    MI_LN_FWD_CASE(3)
+                    MI_LN_FWD_CASE(4)
                     MI_LN_FWD_CASE(16)
                     default: break;
                 }
@@ -915,7 +921,11 @@ int ln_forward_impl(const char* name, const float* a, const float* b, const floa
     }
     const int W = vec4 ? 4 : 1;
     const int need = (cols / W + kWave - 1) / kWave;
-    const int n = pick_n(need);
+    // So do a few rows (at most a wave per SIMD): 4 waves of a quarter row
+    // finish sooner than one (16 rows of 1600, the six forward calls of a
+    // decode step: 28.1 -> 25.8 us; [1000, 2048] fwd + bwd 15.3 -> 14.3 us;
+    // [3000, 1024] would go from 16.3 to 17.7 us).
+    const int n = rows <= kFewRows && need > 1 ? 0 : pick_n(need);
     if (n != 0) {
         const bool two = fwd_rows_per_wave(rows, cols) == 2;
         if (vec4 && two)

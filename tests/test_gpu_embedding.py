@@ -275,3 +275,21 @@ def test_pos_embedding_backward_batch_groups(dev, B, T, D):
     Dwpe = dev_t(dwpe0)
     M.pos_embedding_backward(dev_t(g), Dwpe, B, T, D)
     assert_exact("dwpe", host(Dwpe), O.pos_embedding_backward(g, dwpe0, B, T))
+
+
+# The few-token gather (8192 waves of one 64-vector chunk at most) and the row
+# form past it, with partial chunks, scalar columns and ids out of range.
+@pytest.mark.parametrize("B,T,D", [(1, 1, 4), (16, 1, 1600), (3, 7, 257), (5, 13, 260),
+                                   (8, 1024, 256), (1, 8193, 16), (2, 2048, 512), (2, 2049, 512)])
+def test_embedding_forward_few_tokens(dev, B, T, D):
+    V = 300
+    wte, wpe, ids, _ = emb_inputs(V, D, B, T, B + T)
+    ids[::7] = -1
+    ids[3::11] = V
+    ok = (ids >= 0) & (ids < V)
+    ref = np.where(ok[:, None], wte[np.where(ok, ids, 0)], np.float32(0))
+    out = torch.empty(B * T, D, device=dev)
+    M.embedding_forward(dev_t(wte), dev_t(ids), out, B * T, D, V)
+    assert_exact("embedding_forward", host(out), ref)
+    M.embedding_pos_forward(dev_t(wte), dev_t(wpe), dev_t(ids), out, B, T, D, V)
+    assert_exact("embedding_pos_forward", host(out), O.pos_embedding_forward(wpe, ref, B, T))

@@ -229,10 +229,12 @@ def test_wide_sweep_config4(dev):
 # Edges of the narrow-row kernels (16 and 32 lanes a row, up to 128 columns),
 # of the rows spread over 4 and 16 waves (forward: 16-byte vectors from 4100 columns,
 # scalars from 1025; past 49152 and 12288 the block kernel) and of the scalar
-# backward's vectors per lane, with row counts that leave partial workgroups.
+# backward's vectors per lane, with row counts that leave partial workgroups, and
+# of up to 1024 rows over 4 waves each (forward, past one vector per lane).
 @pytest.mark.parametrize("rows,cols", [
     (1, 4), (17, 60), (1025, 64), (16385, 64), (9, 68), (33, 124), (2049, 128), (40000, 96),
     (65, 132), (19, 1025), (7, 1281), (300, 1538), (5, 4095), (4, 4097), (3, 8191), (2, 8195),
+    (1024, 260), (1025, 260), (2, 1024), (1024, 516), (33, 257), (16, 1600), (1000, 70),
     (3, 12289), (6, 4100), (300, 5120), (3, 12292), (2, 16388), (2, 49156), (700, 640 + 255),
 ])
 def test_layernorm_width_edges(dev, rows, cols):
