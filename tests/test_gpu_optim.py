@@ -139,3 +139,27 @@ def test_adam_past_one_vector_per_thread(dev):
     assert_exact("param", host(P_), po)
     assert_exact("m", host(Mm), mo)
     assert_exact("v", host(V_), vo)
+
+
+# Both sides of the size up to which the Adam pass finishes the norm² itself:
+# the same bits as the separate calls.
+@pytest.mark.parametrize("n", [1, 3, 1025, 262147, (1 << 20) - 3, 1 << 20, (1 << 20) + 1])
+def test_adam_update_equals_its_parts(dev, n):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    grad = torch.randn(n, device="cuda", generator=gen)
+    p0, m0 = torch.randn(n, device="cuda", generator=gen), 0.1 * grad
+    v0 = torch.rand(n, device="cuda", generator=gen)
+    p, m, v = p0.clone(), m0.clone(), v0.clone()
+    norm, clip = torch.full((1,), 7.0, device="cuda"), torch.empty(1, device="cuda")
+    step, scale = 3, 0.5
+    M.adam_update(p, grad, m, v, n, 1e-3, 0.9, 0.999, 1e-8, step, scale, norm, clip)
+    norm2, clip2 = torch.zeros(1, device="cuda"), torch.empty(1, device="cuda")
+    M.buffer_norm_sq_acc(grad, n, norm2)
+    M.compute_clip_scale(norm2, clip2, 1.0 / scale)
+    bc = [float(np.float32(1) - np.float32(np.float32(b) ** np.float32(step))) for b in (0.9, 0.999)]
+    p2, m2, v2 = p0.clone(), m0.clone(), v0.clone()
+    M.adam_clipped(p2, grad, m2, v2, clip2, 1e-3, 0.9, 0.999, 1e-8, bc[0], bc[1], scale, n)
+    for name, a, b in (("norm", norm, norm2), ("clip", clip, clip2), ("m", m, m2), ("v", v, v2),
+                       ("param", p, p2)):
+        assert_exact(name, host(a), host(b))
