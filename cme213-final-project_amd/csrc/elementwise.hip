@@ -314,9 +314,10 @@ __global__ __launch_bounds__(1024) void rowband_kernel(const void* w0, const voi
 // width is no multiple of 4.
 //
 // A row band of one row per workgroup leaves most of the chip idle on narrow
-// rows (one or two waves per CU at 256 or 512 columns: ReLU backward + dbias
-// [8192, 2048] 33 us, [2048, 512] 7.4 us) and falls back to 4-byte accesses
-// where rows do not start on 16 bytes.  Here a workgroup takes RL consecutive
+// rows (one or two waves per CU at 256 or 512 columns) and falls back to
+// 4-byte accesses where rows do not start on 16 bytes.  Memory-bound; half
+// ReLU forward + backward [4096, 1024] 21.8 -> 16.9 us, [16384, 333] 35.8 ->
+// 22.4, [4096, 3002] 46.9 -> 38.4 us.  Here a workgroup takes RL consecutive
 // rows at a time as one contiguous run of sv = RL * cols / 4 vectors, RL a
 // multiple of 4 / gcd(cols, 4), so that every run starts on 16 bytes: thread
 // t owns the super-columns of vectors t + k * T, keeps their biases and sums
@@ -862,7 +863,10 @@ struct LanePlan {
 // Rows of at most 512 vectors take as many row lanes as fill 1024 threads
 // while the runs still go round kLaneBlocks workgroups; wider rows only where
 // their width is no multiple of 4 (one run of 4 or 2 rows, up to 4 vectors
-// per thread).  Rows of 513 to 4096 whole vectors stay with the row bands.
+// per thread).  Rows of 513 to 4096 whole vectors stay with the row bands:
+// GELU backward + dbias by row lanes / by bands [4096, 2048] 20.8 / 21.8 us,
+// [16384, 2048] 68.6 / 72.1, [8192, 1024] 20.6 / 31.0, but [512, 2560] 8.1 /
+// 7.7, [8192, 3072] 52.2 / 51.5, [4096, 8192] 79.2 / 76.9.
 // Below 16 columns the plain bands stay (a run must hold the tail elements'
 // columns, and such rows are never large).
 #ifndef MI_LANE_BLOCKS

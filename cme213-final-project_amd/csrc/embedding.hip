@@ -4,7 +4,8 @@
 // in-place position add, float-atomic scatter-add backward) and the CPU
 // loops of NEW_code/tests/test_embedding.cu:16-41.
 //
-// Forward: one wave per token row, W-wide vector copies; the fused variant
+// Forward: a wave per few token rows, or per row chunk where there are few
+// tokens, W-wide vector copies; the fused variant
 // writes table[id] + pos[t] in one pass (one fp32 add, so bit-identical to
 // the reference's gather followed by its in-place add).
 //
@@ -91,7 +92,8 @@ __global__ __launch_bounds__(kRowWaves * kWave) void emb_fwd_kernel(
 // The gather for few tokens, where the form above leaves most of the chip idle
 // and each wave waits for one row chunk after another (16 tokens of 1600
 // columns: one workgroup, 6.2 us): a wave takes one row's chunk of 64 vectors,
-// so every load of the call is in flight at once.
+// so every load of the call is in flight at once (512 tokens of 320, fwd +
+// bwd, 16.8 -> 8.8 us).
 template <int W, bool POS>
 __global__ __launch_bounds__(kRowWaves * kWave) void emb_fwd_chunk_kernel(
     const float* __restrict__ table, const float* __restrict__ pos, const int* __restrict__ tokens,

@@ -8,9 +8,11 @@
 // Here:
 //  * forward: one wave64 per row, the row held in registers as W-wide
 //    vectors (W = 4 -> global_load_dwordx4), so x is read from HBM once;
-//    mean and variance are two wave reductions over the registers.
-//  * backward: a "row group" of G waves owns a row (G = 1 up to 2048
-//    columns, 4 beyond); grad_out and x are read once per row.  dx is
+//    mean and variance are two wave reductions over the registers.  Rows of
+//    at most 128 columns share a wave; longer rows than one wave holds, and
+//    any row where there are few, are held by 4 or 16 waves.
+//  * backward: a "row group" of G waves owns a row (G = 1 up to 1536
+//    columns, 4 or 8 beyond; rows of at most 128 columns share a wave); grad_out and x are read once per row.  dx is
 //    written in the same pass, and each thread keeps running dgamma/dbeta
 //    sums for the columns it owns across all rows its group visits.  At the
 //    end the groups of a workgroup combine through LDS (fixed tree order)
@@ -181,8 +183,9 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // Forward, a row over the G waves of a workgroup, held in registers: widths
 // past what one wave holds (4096 columns in 16-byte vectors, 1024 in scalars).
 // Memory-bound like the wave kernel; the block kernel below, which these
-// widths took before, walks the row three times in 4-byte accesses ([4096,
-// 5120] fwd + bwd 110 us, [3001, 1026] 23 us).  The statistics cost two LDS
+// widths took before, walks the row three times in 4-byte accesses (fwd + bwd
+// [4096, 5120] 109 -> 84 us, [3001, 1026] 23.3 -> 20.7, [8192, 8192] 331 ->
+// 238 us, 5.6 TB/s).  The statistics cost two LDS
 // exchanges.  gamma and beta of the next vector are requested before the
 // current one is stored: a load behind a store would wait for it (the
 // vector-memory counter retires in order).
@@ -642,7 +645,7 @@ __global__ __launch_bounds__(kBlockThreads) void ln_bwd_block_kernel(
 // Narrow rows (at most 32 16-byte vectors): L = 16 or 32 lanes own a row, one
 // vector per lane, so a wave holds 4 or 2 rows.  With a whole wave per row,
 // half of its lanes or more had no work and each wave kept one short row in
-// flight ([65536, 96] fwd + bwd 48 us).
+// flight ([65536, 96] fwd + bwd 48 -> 28 us, 4.5 TB/s).
 // ---------------------------------------------------------------------------
 
 // Sum over the L lanes of a row, in every one of them; fixed order.
@@ -993,7 +996,7 @@ BwdPlan plan_bwd(int rows, int cols, bool vec4, bool add) {
     // (N = 8 spills).  Scalars hold four times fewer floats per vector, so
     // N goes to 16, which keeps a row on as few waves (with N <= 6, 8 waves
     // of 2 to 6 floats per lane and a barrier per row: [16384, 999] fwd + bwd
-    // 81 us).  Wider rows use the block-per-row kernel.
+    // 81 us against 69).  Wider rows use the block-per-row kernel.
     static const int kG[] = {1, 4, 8};
     static const int kN[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int max_n = p.W == 4 ? 6 : 16;

@@ -13,8 +13,9 @@
 //    after memset + norm + clip kernels.
 //
 // Here the norm² is a deterministic two-pass sum (per-workgroup partials in
-// the library workspace, then one workgroup adding them in a fixed order,
-// which can also derive the clip scale), and Adam is one grid-stride pass of
+// the library workspace, then one workgroup, or for few parameters every
+// workgroup of the Adam pass, adding them in a fixed order and deriving the
+// clip scale), and Adam is one grid-stride pass of
 // 16-byte vectors.  The Adam arithmetic is evaluated exactly as written
 // (no FMA contraction), so it is bit-identical to the CPU statement of the
 // reference kernel given the same clip scale.

@@ -11,8 +11,8 @@
 //  * cross_entropy_forward_v2 (:517-532): scale 1 / batch; the mean loss
 //    stays on the device (memset + atomicAdd tree + a divide kernel).
 //
-// Here a "row group" of G waves holds a row in registers (K elements per
-// lane), so the row is read from HBM once and the output written once.  The
+// Here a "row group" of G waves holds a row in registers (K accesses of
+// 4 or 16 bytes per lane), so the row is read from HBM once and the output written once.  The
 // row maximum and sum are wave reductions (DPP) combined across the G waves
 // in a fixed order through LDS.  Rows longer than 65536 use a block-per-row
 // kernel that streams the row three times, as the reference does.  The
