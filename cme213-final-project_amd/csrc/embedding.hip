@@ -625,11 +625,15 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
                     const unsigned long long m = __ballot(bit);
                     same &= bit ? m : ~m;
                 }
-                if (ok) {
-                    int* const c = &cnt[wave * kBins + static_cast<int>(num)];
-                    at[q] = *c + __popcll(same & below);
-                    if ((same & below) == 0ull) *c += __popcll(same);
-                }
+                int* const c = &cnt[wave * kBins + static_cast<int>(num)];
+                const int upto = ok ? *c : 0;
+                at[q] = upto + __popcll(same & below);
+                // The counts pass between the wave's lanes: every lane has
+                // read its count before the lowest equal lane updates it, and
+                // the update is made before the next group reads.
+                wave_order();
+                if (ok && (same & below) == 0ull) *c = upto + __popcll(same);
+                wave_order();
             }
             __syncthreads();
             // Thread t takes the numbers t * kPer + [0, kPer).

@@ -142,6 +142,15 @@ __device__ __forceinline__ void store16(uint16_t* base, size_t vec_index, const 
 
 inline bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 
+// Orders LDS accesses between the lanes of one wave: what a lane accessed
+// before the call comes before what any lane accesses after it.  The hardware
+// runs a wave's LDS accesses in program order, so this only keeps the
+// compiler from moving them (no instruction is emitted).
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // ---------------------------------------------------------------------------
 // Wave64 sum.  Four DPP steps reduce each 16-lane row (quad xor-1, quad
 // xor-2, half-row mirror, row mirror); the four row totals are then read
