@@ -210,6 +210,19 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(readlane(v, 0), readlane(v, 16)), fmaxf(readlane(v, 32), readlane(v, 48)));
 }
 
+// Wave64 bitwise OR with the same DPP pattern; every lane returns the result.
+// All 64 lanes must be active.
+__device__ __forceinline__ unsigned wave_or(unsigned v) {
+    v |= __float_as_uint(dpp_move<0xB1>(__uint_as_float(v)));
+    v |= __float_as_uint(dpp_move<0x4E>(__uint_as_float(v)));
+    v |= __float_as_uint(dpp_move<0x141>(__uint_as_float(v)));
+    v |= __float_as_uint(dpp_move<0x140>(__uint_as_float(v)));
+    const int x = static_cast<int>(v);
+    return static_cast<unsigned>(
+        (__builtin_amdgcn_readlane(x, 0) | __builtin_amdgcn_readlane(x, 16)) |
+        (__builtin_amdgcn_readlane(x, 32) | __builtin_amdgcn_readlane(x, 48)));
+}
+
 // ---------------------------------------------------------------------------
 // Host plumbing (defined in runtime.hip).
 // ---------------------------------------------------------------------------
