@@ -317,7 +317,7 @@ __global__ __launch_bounds__(1024) void rowband_kernel(const void* w0, const voi
 // rows (one or two waves per CU at 256 or 512 columns) and falls back to
 // 4-byte accesses where rows do not start on 16 bytes.  Memory-bound; half
 // ReLU forward + backward [4096, 1024] 21.8 -> 16.9 us, [16384, 333] 35.8 ->
-// 22.4, [4096, 3002] 46.9 -> 38.4 us.  Here a workgroup takes RL consecutive
+// 22.4 us.  Here a workgroup takes RL consecutive
 // rows at a time as one contiguous run of sv = RL * cols / 4 vectors, RL a
 // multiple of 4 / gcd(cols, 4), so that every run starts on 16 bytes: thread
 // t owns the super-columns of vectors t + k * T, keeps their biases and sums
@@ -860,28 +860,29 @@ struct LanePlan {
     int rl = 0, nc = 0, threads = 0, sv = 0, blocks = 0;
 };
 
-// Rows of at most 512 vectors take as many row lanes as fill 1024 threads
-// while the runs still go round kLaneBlocks workgroups; wider rows only where
-// their width is no multiple of 4 (one run of 4 or 2 rows, up to 4 vectors
-// per thread).  Rows of 513 to 4096 whole vectors stay with the row bands:
-// GELU backward + dbias by row lanes / by bands [4096, 2048] 20.8 / 21.8 us,
-// [16384, 2048] 68.6 / 72.1, [8192, 1024] 20.6 / 31.0, but [512, 2560] 8.1 /
-// 7.7, [8192, 3072] 52.2 / 51.5, [4096, 8192] 79.2 / 76.9.
+// Rows take as many row lanes as fill 1024 threads while the runs still go
+// round kLaneBlocks workgroups, up to 2048 columns, and up to kLaneRagged where
+// the width is no multiple of 4.  Wider rows stay with the row bands: GELU
+// backward + dbias by row lanes / by bands [4096, 2048] 20.8 / 21.8 us, [16384,
+// 2048] 68.6 / 72.1, [8192, 1024] 20.6 / 31.0, but [512, 2560] 8.1 / 7.7, [8192,
+// 3072] 52.2 / 51.5, [4096, 8192] 79.2 / 76.9.  Ragged widths, lanes over bands in
+// time, tensors in the last-level cache / in HBM: [8192, 999] 0.99 / 0.70, [8192,
+// 1101] 0.98 / 0.71, [8192, 1201] 1.05 / 0.76, [8192, 1538] 1.09 / 0.85, [4096, 1701]
+// 1.19 / 0.98, [4096, 2302] 1.15 / 0.99, [1000, 4094] 1.32 / 1.10, [256, 8190] 1.78 /
+// 1.65: a run of one row unit leaves a CU one workgroup with one to four
+// vectors a thread in flight (two runs in flight: 1.0 to 1.1 times slower).
 // Below 16 columns the plain bands stay (a run must hold the tail elements'
 // columns, and such rows are never large).
-#ifndef MI_LANE_BLOCKS
-#define MI_LANE_BLOCKS 256
-#endif
-#ifndef MI_LANE_THREADS
-#define MI_LANE_THREADS 1024
-#endif
-constexpr int kLaneBlocks = MI_LANE_BLOCKS;
-constexpr int kLaneThreads = MI_LANE_THREADS;
+constexpr int kLaneBlocks = 256;
+constexpr int kLaneThreads = 1024;
+constexpr int kLaneRagged = 1152;
+constexpr int kLaneNC = 2;  // vectors per thread: 4 rows of kLaneRagged columns at most
+static_assert(kLaneRagged <= kLaneNC * 1024, "the widest run fits the threads");
 
 LanePlan plan_lanes(int rows, int cols) {
     LanePlan p;
     const int unit = cols % 4 == 0 ? 1 : cols % 2 == 0 ? 2 : 4;  // rows of a 16-byte aligned run
-    if (cols < 16 || cols > kMaxNC * 4096 / unit || (unit == 1 && cols > 2048)) return p;
+    if (cols < 16 || cols > (unit == 1 ? 2048 : kLaneRagged)) return p;
     const int sv1 = unit * cols / 4;
     int m = kLaneThreads / sv1;  // units per run
     const int most = rows / (unit * kLaneBlocks);
@@ -916,8 +917,6 @@ int launch_rowlane_reduce(const char* name, const LanePlan& p, Op op, const floa
     switch (p.nc) {
         MI_LANE_CASE(1)
         MI_LANE_CASE(2)
-        MI_LANE_CASE(3)
-        MI_LANE_CASE(4)
         default:
             break;
     }
