@@ -46,20 +46,18 @@ constexpr int sm_threads() {
     return (G < 4 ? 4 : G) * kWave;
 }
 
-// V = 4 takes 16-byte accesses (cols % 4 == 0 and 16-byte aligned tensors), V
-// = 1 4-byte ones; K accesses per lane.
+// V = 4 takes 16-byte accesses, V = 1 4-byte ones; K accesses per lane.
 //
-// Memory-bound.  16-byte stores carry the non-temporal hint, and rows over 8
-// waves or more (past 2048 columns) load with it too; [16384, 1024] softmax 34.8 -> 21.0
-// us (28.7 without the hint, 24.8 with it on the loads too), [16384, 1100]
-// 51.5 -> 23.1, [4096, 32000] 195 -> 176 (181 with stores alone), cross-entropy
-// [8192, 32000] 374 -> 348.  4-byte accesses do better without: their rows
-// start anywhere, and lines shared by two waves are then written twice.
-// Sharing one long row between workgroups that each read all of it and store
-// a part was slower ([64, 32000] 7.1 -> 8.8 us, 16 rows of 50257 9.4 -> 21).
+// Memory-bound.  16-byte stores carry the non-temporal hint: [16384, 1024]
+// softmax 34.7 -> 26.3 us, [16384, 1100] 51.7 -> 27.1, [4096, 32000] 194 -> 180,
+// cross-entropy [8192, 32000] 373 -> 360 (180 -> 173 and 360 -> 344 with it on
+// the loads too, see stream_rows).  4-byte accesses do better without: their
+// rows start anywhere, and lines shared by two waves are then written twice.
+// Sharing one long row between workgroups that each read all of it and store a
+// part was slower ([64, 32000] 7.1 -> 8.8 us, 16 rows of 50257 9.4 -> 21).
 constexpr int kNontemporal = 2;  // cache-policy bit of the buffer accesses
 
-template <int G, int K, bool CE, int V>
+template <int G, int K, bool CE, int V, bool NT>
 __global__ __launch_bounds__(sm_threads<G>()) void row_softmax_kernel(
     const float* __restrict__ x, float* __restrict__ out, int rows, int cols,
     const int* __restrict__ targets, float* __restrict__ losses, float scale) {
@@ -89,7 +87,7 @@ __global__ __launch_bounds__(sm_threads<G>()) void row_softmax_kernel(
     for (int k = 0; k < K; ++k) {
         if constexpr (V == 4) {
             const auto a = __builtin_amdgcn_raw_buffer_load_b128(rin, t * 16, k * GT * 16,
-                                                                 G >= 8 ? kNontemporal : 0);
+                                                                 NT ? kNontemporal : 0);
             const bool ok = 4 * (t + k * GT) < cols;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[k][e] = ok ? __int_as_float(a[e]) : -FLT_MAX;
@@ -281,19 +279,43 @@ SmPlan plan_softmax(int cols, bool vec4) {
     return {};
 }
 
+// Whether the loads of rows over 8 waves or more (past 4096 columns) carry the
+// hint too: where the logits are half as large again as the 256 MB last-level
+// cache, so that they come from memory, and rows past 49152 columns.  Time of
+// the hinted form over the plain one's, logits from memory / in the cache: [4096,
+// 8192] 0.94 / 1.09, [4096, 16384] 0.96 / 1.15, [2048, 32000] 0.97 / 1.14, [1000, 32000]
+// 0.95 / 1.11, but [4096, 32000] 0.96 and [8192, 32000] 0.95 always, [256, 50304]
+// 0.95 / 0.91, [300, 64000] 0.97 / 1.00, [512, 65536] 0.92 / 1.04.  The longest rows
+// gain over 4-byte accesses except where one or two fall to each CU and the
+// logits are in the cache (65536 columns: 64 rows 0.72 / 0.63, 256 rows 0.98 / 1.14,
+// 512 rows 0.94 / 1.20, 768 rows 0.91 / 0.89).
+bool stream_rows(int rows, int cols) {
+    return cols > 49152 || static_cast<long long>(rows) * cols > (3ll << 25);
+}
+
 template <int G, int K, bool CE, int V>
 void launch_rows(int rows, int cols, hipStream_t st, const float* x, float* out, const int* tg,
                  float* losses, float scale) {
     constexpr int GPB = G < 4 ? 4 / G : 1;
     const dim3 grid(static_cast<unsigned>((static_cast<long long>(rows) + GPB - 1) / GPB));
-    hipLaunchKernelGGL((row_softmax_kernel<G, K, CE, V>), grid, dim3(sm_threads<G>()), 0, st, x,
-                       out, rows, cols, tg, losses, scale);
+    if constexpr (V == 4 && G >= 8) {
+        if (stream_rows(rows, cols)) {
+            hipLaunchKernelGGL((row_softmax_kernel<G, K, CE, V, true>), grid,
+                               dim3(sm_threads<G>()), 0, st, x, out, rows, cols, tg, losses, scale);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((row_softmax_kernel<G, K, CE, V, false>), grid, dim3(sm_threads<G>()), 0,
+                       st, x, out, rows, cols, tg, losses, scale);
 }
 
 template <bool CE>
 void launch_softmax(int rows, int cols, hipStream_t st, const float* x, float* out, const int* tg,
                     float* losses, float scale) {
-    const bool vec4 = cols % 4 == 0 && aligned16(x) && aligned16(out);
+    // Up to 64 columns a 4-byte access already holds the row, and a 16-byte one
+    // leaves most lanes idle: its time over the other's, 65536 rows of 16, 32, 64,
+    // 68, 96 columns, 1.16, 1.11, 1.05, 0.85, 0.80.
+    const bool vec4 = cols > 64 && cols % 4 == 0 && aligned16(x) && aligned16(out);
     const SmPlan p = plan_softmax(cols, vec4);
 #define MI_SM_CASE(GG, KK, VV)                                                  \
     if (p.G == GG && p.K == KK && vec4 == (VV == 4)) {                           \

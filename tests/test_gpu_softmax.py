@@ -160,11 +160,36 @@ def test_model_size_cross_entropy(dev):
 @pytest.mark.parametrize("rows,cols", [
     (5, 252), (9, 256), (3, 260), (7, 1020), (5, 1028), (3, 1540), (3, 2052), (2, 4100),
     (2, 8196), (3, 12292), (2, 28676), (1, 65532), (1, 65540),
+    (7, 64), (9, 68),
     (5, 385), (6, 641), (3, 1025), (3, 1281), (2, 2561), (3, 5121), (2, 9217), (1, 40961),
 ])
 def test_row_shape_edges(dev, rows, cols):
     test_softmax_shapes(dev, rows, cols)
     test_cross_entropy_shapes_v1_and_v2(dev, rows, cols)
+
+
+# Logits past the size from which they are loaded with the streaming hint: the
+# same bits as the first rows alone, which are not.
+@pytest.mark.parametrize("cols", [4100, 49152])
+def test_large_logits_equal_their_first_rows(dev, cols):
+    rows = (3 << 25) // cols + 1
+    note(f"softmax and cross_entropy {rows}x{cols}")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(cols)
+    x = torch.randn(rows, cols, device="cuda", generator=gen)
+    t = torch.randint(0, cols, (rows,), device="cuda", generator=gen, dtype=torch.int32)
+    y, losses, lout = torch.empty_like(x), torch.empty(rows, device="cuda"), torch.empty(1, device="cuda")
+    z, few = torch.empty(64, cols, device="cuda"), torch.empty(64, device="cuda")
+    M.softmax_forward(x, y, rows, cols)
+    M.softmax_forward(x[:64], z, 64, cols)
+    assert_exact("softmax", host(y[:64]), host(z))
+    assert bool(((y.sum(1, dtype=torch.float64) - 1).abs() < 1e-5).all())
+    M.cross_entropy_forward(x, t, y, rows, cols)          # gradient not scaled by the batch
+    M.cross_entropy_forward(x[:64], t[:64], z, 64, cols)
+    assert_exact("cross-entropy gradient", host(y[:64]), host(z))
+    M.cross_entropy_forward_v2(x, t, y, losses, lout, rows, cols)
+    M.cross_entropy_forward_v2(x[:64], t[:64], z, few, lout, 64, cols)
+    assert_exact("losses", host(losses[:64]), host(few))
 
 
 def test_unaligned_rows_take_the_scalar_accesses(dev):
@@ -178,3 +203,33 @@ def test_unaligned_rows_take_the_scalar_accesses(dev):
     Z = dev_t(x)
     M.softmax_forward(Z, Z, rows, cols)   # in place
     assert_fwd("softmax, in place", host(Z), O.softmax_forward_f64(x))
+
+
+def _us(call, n=60):
+    """Microseconds per call, the least of seven batches of n."""
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = float("inf")
+    for _ in range(8):  # the first one warms up
+        torch.cuda.synchronize()
+        a.record()
+        for _ in range(n):
+            call()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best
+
+
+# Tensors off 16 bytes take 4-byte accesses, the general path; on 16 bytes no
+# shape is slower than that.
+@pytest.mark.parametrize("rows,cols", [(65536, 16), (4096, 8192)])
+def test_softmax_time_against_the_scalar_accesses(dev, rows, cols):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(cols)
+    n = rows * cols
+    x, y = torch.randn(n + 1, device="cuda", generator=gen), torch.empty(n + 1, device="cuda")
+    t = [_us(M.bind("mi_softmax_forward", x[o:o + n], y[o:o + n], rows, cols)) for o in (0, 1)]
+    note(f"softmax [{rows}, {cols}]: {t[0]:.2f} us, {t[1]:.2f} us off 16 bytes")
+    # 0.99 measured; 1.18 and 1.08 with 16-byte accesses at every width and the
+    # streaming hint on the loads of every row past 4096 columns
+    assert t[0] <= 1.06 * t[1]
