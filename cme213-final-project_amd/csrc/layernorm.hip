@@ -495,8 +495,10 @@ __global__ __launch_bounds__(NWV * kWave) void ln_bwd_group_kernel(
     // and at most 2 vectors per lane, two rows in flight were faster ([8192,
     // 1600]: 34.0 against 36.7 us; [32768, 1600]: 109.0 against 124.1 us);
     // with 4 vectors per lane the second row costs occupancy ([32768, 4096]:
-    // 290 against 269 us).
-    constexpr int RF = (G > 1 && N * W <= 8) ? 2 : 1;
+    // 290 against 269 us), and so it does with 6 or 8 scalars ([16384, 1302]:
+    // 51.7 against 47.7 us; residual form [16384, 1026] 47.7 against 45.1, [4096,
+    // 1802] 24.3 against 22.5).
+    constexpr int RF = (G > 1 && N <= 2) ? 2 : 1;
     const int first = blockIdx.x * GPB;
     const unsigned iters = strided_trips(static_cast<unsigned>(first), static_cast<unsigned>(rows),
                                          static_cast<unsigned>(stride));
@@ -996,7 +998,10 @@ BwdPlan plan_bwd(int rows, int cols, bool vec4, bool add) {
     // (N = 8 spills).  Scalars hold four times fewer floats per vector, so
     // N goes to 16, which keeps a row on as few waves (with N <= 6, 8 waves
     // of 2 to 6 floats per lane and a barrier per row: [16384, 999] fwd + bwd
-    // 81 us against 69).  Wider rows use the block-per-row kernel.
+    // 81 us against 69; the residual form gains at 771 columns, [16384, 771]
+    // 42.6 against 47.8 us, and at 1001 only where the tensors are in the
+    // last-level cache: [16384, 1001] 41.8 against 43.1, from memory 56.0
+    // against 52.4).  Wider rows use the block-per-row kernel.
     static const int kG[] = {1, 4, 8};
     static const int kN[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int max_n = p.W == 4 ? 6 : 16;
