@@ -214,15 +214,19 @@ __global__ __launch_bounds__(G * kWave) void ln_fwd_group_kernel(
             for (int e = 0; e < W; ++e) v[k].v[e] = v[k].v[e] + w.v[e];
         }
     }
-    // Sum over the row's waves, in wave order; every thread gets it.
+    // Sum over the row's waves, pairwise; every thread gets it.
     auto row_sum = [&](float x, int slot) __attribute__((always_inline)) {
         const float w = wave_sum(x);
         if ((t & (kWave - 1)) == 0) red[slot][wave] = w;
         __syncthreads();
-        float r = red[slot][0];
+        float r[G];
 #pragma unroll
-        for (int i = 1; i < G; ++i) r += red[slot][i];
-        return r;
+        for (int i = 0; i < G; ++i) r[i] = red[slot][i];
+#pragma unroll
+        for (int h = G / 2; h >= 1; h /= 2)
+#pragma unroll
+            for (int i = 0; i < h; ++i) r[i] += r[i + h];
+        return r[0];
     };
     float s = 0.0f;
 #pragma unroll
@@ -707,10 +711,14 @@ __global__ __launch_bounds__(kBlockThreads) void ln_fwd_sub_kernel(
     }
 }
 
-// Backward, T threads per workgroup (T / L rows at a time), RF rows per lane
-// group in flight; the groups' sums are staged in LDS as [2 * cols] rows and
-// added in group order into the workgroup's partial row.
+// Backward, T threads per workgroup (T / L rows at a time), kSubRows rows per
+// lane group in flight; the groups' sums are staged in LDS as [2 * cols] rows
+// and added into the workgroup's partial row as kSubSums interleaved sums, then
+// pairwise.  (One sum in group order, up to 64 terms in sequence, had a larger
+// rounding error than a wave per row: dbeta of [65536, 64], relative 2-norm
+// against float64, 2.0e-7 against 1.5e-7; 1.3e-7 so.)
 constexpr int kSubRows = 2;
+constexpr int kSubSums = 8;  // divides the number of groups: 8 to 64, a power of two
 
 template <int L, bool ADD>
 __global__ __launch_bounds__(1024) void ln_bwd_sub_kernel(
@@ -786,9 +794,17 @@ __global__ __launch_bounds__(1024) void ln_bwd_sub_kernel(
     __syncthreads();
     float* prow = part + static_cast<size_t>(blockIdx.x) * 2 * cols;
     for (int c = threadIdx.x; c < 2 * cols; c += T) {
-        float t = sub_sums[c];
-        for (int i = 1; i < gpb; ++i) t += sub_sums[i * 2 * cols + c];
-        prow[c] = t;
+        float t[kSubSums];
+#pragma unroll
+        for (int i = 0; i < kSubSums; ++i) t[i] = sub_sums[i * 2 * cols + c];
+        for (int g = kSubSums; g < gpb; g += kSubSums)
+#pragma unroll
+            for (int i = 0; i < kSubSums; ++i) t[i] += sub_sums[(g + i) * 2 * cols + c];
+#pragma unroll
+        for (int h = kSubSums / 2; h >= 1; h /= 2)
+#pragma unroll
+            for (int i = 0; i < h; ++i) t[i] += t[i + h];
+        prow[c] = t[0];
     }
 }
 
@@ -985,7 +1001,7 @@ BwdPlan plan_bwd(int rows, int cols, bool vec4, bool add) {
         while (p.waves > 4 && static_cast<long long>(p.waves) * kWave / p.lanes *
                                       MI_LN_BWD_MAX_BLOCKS > rows)
             p.waves /= 2;
-        const int gpb = p.waves * kWave / p.lanes;
+        const int gpb = p.waves * kWave / p.lanes;  // 8 to 64: a multiple of kSubSums
         const long long groups = (static_cast<long long>(rows) + gpb - 1) / gpb;
         p.blocks = static_cast<int>(groups < MI_LN_BWD_MAX_BLOCKS ? groups : MI_LN_BWD_MAX_BLOCKS);
         if (p.blocks < 1) p.blocks = 1;
