@@ -41,3 +41,21 @@ def gelu_inputs(rows, cols, seed):
     b = (0.02 * r.standard_normal(cols)).astype(np.float32)
     g = r.standard_normal((rows, cols), dtype=np.float32)
     return x, b, g
+
+
+def batch_us(*calls, n=60):
+    """Microseconds per call of each: the least of ten batches of n, the calls'
+    batches in turn, so that all of them see the same states of the machine."""
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = [float("inf")] * len(calls)
+    for rep in range(11):
+        for i, call in enumerate(calls):
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(n):
+                call()
+            b.record()
+            torch.cuda.synchronize()
+            if rep:  # the first round warms up
+                best[i] = min(best[i], a.elapsed_time(b) * 1e3 / n)
+    return best

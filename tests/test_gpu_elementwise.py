@@ -7,7 +7,7 @@ import torch
 
 import cme213_amd as M
 import oracle as O
-from gpu_util import dev_t, gelu_inputs, host, note
+from gpu_util import batch_us, dev_t, gelu_inputs, host, note
 from tol import (assert_bwd, assert_bwd_within_oracle_error, assert_colsum, assert_exact,
                  assert_fwd, assert_fwd_within_oracle_error)
 
@@ -249,21 +249,6 @@ def test_column_sums_row_lanes(dev, rows, cols, off):
     assert_colsum("gelu dbias", host(DB), db64 + db0.astype(np.float64), gin64, approx_terms=True)
 
 
-def _us(call, n=60):
-    """Microseconds per call, the least of seven batches of n."""
-    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    best = float("inf")
-    for _ in range(8):  # the first one warms up
-        torch.cuda.synchronize()
-        a.record()
-        for _ in range(n):
-            call()
-        b.record()
-        torch.cuda.synchronize()
-        best = min(best, a.elapsed_time(b) * 1e3 / n)
-    return best
-
-
 # Tensors off 16 bytes take the row bands with 4-byte accesses, the general
 # path; on 16 bytes no width is slower than that.
 @pytest.mark.parametrize("rows,cols", [(4096, 999), (1500, 2050), (1000, 4094), (256, 8190)])
@@ -273,8 +258,8 @@ def test_gelu_backward_ragged_widths_time(dev, rows, cols):
     n = rows * cols
     bias, db = torch.randn(cols, device=dev, generator=gen), torch.zeros(cols, device=dev)
     x, g, gin = (torch.randn(n + 1, device=dev, generator=gen) for _ in range(3))
-    t = [_us(M.bind("mi_gelu_backward_with_bias_backward", x[o:o + n], bias, g[o:o + n],
-                    gin[o:o + n], db, rows, cols)) for o in (0, 1)]
+    t = batch_us(*(M.bind("mi_gelu_backward_with_bias_backward", x[o:o + n], bias, g[o:o + n],
+                          gin[o:o + n], db, rows, cols) for o in (0, 1)))
     note(f"gelu backward [{rows}, {cols}]: {t[0]:.2f} us, {t[1]:.2f} us off 16 bytes")
     # at most 1.0 measured; 1.2 to 1.8 with row lanes at every ragged width
     assert t[0] <= 1.15 * t[1]

@@ -9,7 +9,7 @@ import torch
 
 import cme213_amd as M
 import oracle as O
-from gpu_util import dev_t, host, note
+from gpu_util import batch_us, dev_t, host, note
 from tol import assert_exact
 
 pytestmark = pytest.mark.gpu
@@ -274,21 +274,6 @@ def test_embedding_backward_run_lengths(dev, V, D, n, lengths, vocab_arg):
     assert_exact("fused dwpe", host(Fwpe), O.pos_embedding_backward(g, dwpe0, 1, n))
 
 
-def _us(call, n=100):
-    """Microseconds per call, the least of seven batches of n."""
-    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    best = float("inf")
-    for _ in range(8):  # the first one warms up
-        torch.cuda.synchronize()
-        a.record()
-        for _ in range(n):
-            call()
-        b.record()
-        torch.cuda.synchronize()
-        best = min(best, a.elapsed_time(b) * 1e3 / n)
-    return best
-
-
 # The vocabulary bound is a check, not a hint: without it (the form of the C++
 # drop-in entry point) the ids are the same, and so is the work.
 @pytest.mark.parametrize("n,V", [(16, 50257), (8192, 5000), (16384, 50257)])
@@ -299,10 +284,11 @@ def test_embedding_backward_time_without_vocabulary_bound(dev, n, V):
     g = torch.randn(n, D, device=dev, generator=gen)
     ids = torch.randint(0, V, (n,), device=dev, generator=gen, dtype=torch.int32)
     dwte = torch.zeros(V, D, device=dev)
-    t = {v: _us(M.bind("mi_embedding_backward", g, ids, dwte, n, D, v)) for v in (V, 0)}
-    note(f"embedding backward n={n} V={V}: {t[V]:.2f} us bounded, {t[0]:.2f} us without a bound")
+    with_bound, without = batch_us(*(M.bind("mi_embedding_backward", g, ids, dwte, n, D, v)
+                                     for v in (V, 0)))
+    note(f"embedding backward n={n} V={V}: {with_bound:.2f} us, {without:.2f} us without a bound")
     # 1.02 to 1.06 measured; 1.34 to 2.4 where every list was sorted bit by bit
-    assert t[0] <= 1.2 * t[V]
+    assert without <= 1.2 * with_bound
 
 
 @pytest.mark.parametrize("B,T,D", [(1, 3, 5), (7, 5, 64), (8, 4, 64), (9, 4, 128), (17, 3, 33)])

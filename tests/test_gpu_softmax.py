@@ -17,7 +17,7 @@ import torch
 
 import cme213_amd as M
 import oracle as O
-from gpu_util import dev_t, host, note
+from gpu_util import batch_us, dev_t, host, note
 from tol import assert_bwd, assert_exact, assert_fwd, assert_fwd_within_oracle_error
 
 pytestmark = pytest.mark.gpu
@@ -205,21 +205,6 @@ def test_unaligned_rows_take_the_scalar_accesses(dev):
     assert_fwd("softmax, in place", host(Z), O.softmax_forward_f64(x))
 
 
-def _us(call, n=60):
-    """Microseconds per call, the least of seven batches of n."""
-    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    best = float("inf")
-    for _ in range(8):  # the first one warms up
-        torch.cuda.synchronize()
-        a.record()
-        for _ in range(n):
-            call()
-        b.record()
-        torch.cuda.synchronize()
-        best = min(best, a.elapsed_time(b) * 1e3 / n)
-    return best
-
-
 # Tensors off 16 bytes take 4-byte accesses, the general path; on 16 bytes no
 # shape is slower than that.
 @pytest.mark.parametrize("rows,cols", [(65536, 16), (4096, 8192)])
@@ -228,7 +213,8 @@ def test_softmax_time_against_the_scalar_accesses(dev, rows, cols):
     gen.manual_seed(cols)
     n = rows * cols
     x, y = torch.randn(n + 1, device="cuda", generator=gen), torch.empty(n + 1, device="cuda")
-    t = [_us(M.bind("mi_softmax_forward", x[o:o + n], y[o:o + n], rows, cols)) for o in (0, 1)]
+    t = batch_us(*(M.bind("mi_softmax_forward", x[o:o + n], y[o:o + n], rows, cols)
+                   for o in (0, 1)))
     note(f"softmax [{rows}, {cols}]: {t[0]:.2f} us, {t[1]:.2f} us off 16 bytes")
     # 0.99 measured; 1.18 and 1.08 with 16-byte accesses at every width and the
     # streaming hint on the loads of every row past 4096 columns
