@@ -28,6 +28,7 @@ namespace {
 constexpr int kOptThreads = 256;
 constexpr int kNormBlocks = 1024;  // partial sums of the norm² pass
 constexpr int kFinThreads = 1024;
+static_assert(kNormBlocks <= kFinThreads, "sum_partials takes one partial a thread");
 
 // ----- sum of squares --------------------------------------------------------
 
@@ -189,10 +190,14 @@ __global__ __launch_bounds__(kOptThreads) void scale_kernel(float* __restrict__ 
     }
 }
 
-// Parameters up to which the Adam pass finishes the norm itself: 20,001 to
-// 600,000 13.4 -> 10.6 us a call, 2 million 15.8 us both ways, 6 million 36.3
-// against 37.2.
+// Parameters up to which the Adam pass finishes the norm itself, and its
+// workgroups, each of which reads all the partials (one thread per vector, or
+// per parameter where n is no multiple of 4).  Separate / fused: 20,001 to
+// 300,001 parameters 10.4 / 8.1 us a call, 600,001 10.3 / 9.3, 800,001 10.5 / 10.3,
+// 1,000,001 10.2 / 11.2; 1,000,000 10.2 / 9.6, 2 million 13.9 / 14.0, 6 million 36.3 /
+// 37.2.
 constexpr long long kFusedParams = 1 << 20;
+constexpr long long kFusedBlocks = 2560;
 
 unsigned flat_grid(long long nvec, int cap) {
     long long g = (nvec + kOptThreads - 1) / kOptThreads;
@@ -235,6 +240,11 @@ int sumsq_impl(const char* name, const float* buf, long long n, float* result, b
     return check_launch(name);
 }
 
+bool adam_vec4(const float* param, const float* grad, const float* m, const float* v,
+               long long n) {
+    return n % 4 == 0 && aligned16(param) && aligned16(grad) && aligned16(m) && aligned16(v);
+}
+
 int adam_impl(const char* name, float* param, const float* grad, float* m, float* v,
               const float* clip, const AdamArgs& a, long long n, hipStream_t st,
               const NormPart* np = nullptr) {
@@ -242,8 +252,7 @@ int adam_impl(const char* name, float* param, const float* grad, float* m, float
     if (n == 0) return MI_OK;
     if (!param || !grad || !m || !v || !clip)
         return set_error(MI_ERR_INVALID_ARG, "%s: NULL pointer", name);
-    const bool vec4 = n % 4 == 0 && aligned16(param) && aligned16(grad) && aligned16(m) &&
-                      aligned16(v);
+    const bool vec4 = adam_vec4(param, grad, m, v, n);
     const long long nvec = vec4 ? n / 4 : n;
     const dim3 grid(flat_grid(nvec, kAdamGrid));
     const NormPart none{};
@@ -319,9 +328,11 @@ int mi_adam_update(float* param, const float* grad, float* m, float* v, long lon
     const float bc2 = 1.0f - powf(beta2, static_cast<float>(step));
     const float max_norm = (grad_scale > 0.0f) ? (1.0f / grad_scale) : 1.0f;
     // The reference zeroes *d_norm_sq with a memset and accumulates into it;
-    // here the finalize overwrites it, so no memset node is needed.  Up to
-    // kFusedParams parameters the Adam pass does the finalize's work.
-    const bool fused = n > 0 && n <= kFusedParams && param && m && v;
+    // here the finalize overwrites it, so no memset node is needed.  With few
+    // parameters the Adam pass does the finalize's work.
+    const long long nvec = adam_vec4(param, grad, m, v, n) ? n / 4 : n;
+    const bool fused = n > 0 && n <= kFusedParams && nvec <= kFusedBlocks * kOptThreads && param &&
+                       m && v;
     NormPart np{};
     int rc = sumsq_impl(name, grad, n, d_norm_sq, false, d_clip_scale, max_norm, st,
                         fused ? &np : nullptr);
