@@ -994,10 +994,14 @@ extern "C" {
 
 size_t mi_bias_backward_workspace(int rows, int cols) {
     if (rows <= 0 || cols <= 0) return 0;
-    // the vec4 and scalar plans can differ; report the larger
-    const size_t a = colsum_bytes(plan_reduce_parts(rows, cols / 4), cols);
-    const size_t b = colsum_bytes(plan_reduce_parts(rows, cols), cols);
-    return a > b ? a : b;
+    // the band plans of 16-byte and 4-byte accesses and the row-lane plan can
+    // differ; report the largest
+    int parts = plan_lanes(rows, cols).blocks;
+    for (int nv : {cols / 4, cols}) {
+        const int p = plan_reduce_parts(rows, nv);
+        if (p > parts) parts = p;
+    }
+    return colsum_bytes(parts, cols);
 }
 
 int mi_residual_add(const float* a, const float* b, float* out, long long n, void* stream) {

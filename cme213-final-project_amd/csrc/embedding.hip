@@ -11,10 +11,13 @@
 //
 // Token backward, deterministic and bit-identical to the CPU loop, which
 // adds grad rows into grad_table in increasing token position: one kernel,
-// no sort and no workspace (emb_bwd_owner_kernel below).  Each workgroup
-// owns a slice of the ids, collects the positions of its ids from the
-// whole id vector, sorts them by id in LDS and adds every id's rows in
-// position order; exactly one wave updates a given table row.
+// no workspace (emb_bwd_owner_kernel below).  The ids are split into classes
+// and each class belongs to a few workgroups, every one of which collects
+// the positions of the class's ids from the whole id vector and sorts them by
+// id in LDS.  Each element (table row, column) has exactly one workgroup that
+// updates it in a call, in position order: a row's columns are shared out
+// over the class's workgroups where the id is frequent or the class's list
+// does not fit LDS at once, and go to one workgroup otherwise.
 // Position backward: one thread per (t, column vector) adds grad_out[b, t]
 // for b = 0, 1, ... in order onto grad_pos[t]; the fused token + position
 // backward does the same sums inside the token kernel's workgroups.
@@ -200,28 +203,26 @@ constexpr int kOwnPerSmall = 8;                  // the same for small token cou
 constexpr int kOwnCap = 2048;                    // list entries per window
 constexpr int kOwnTake = 2;                      // sorted entries per claim
 constexpr int kOwnMaxGrid = 512;                 // workgroups, at most
-#ifndef MI_OWN_LOG2S
-#define MI_OWN_LOG2S 2
-#endif
-#ifndef MI_OWN_LIST
-#define MI_OWN_LIST 256
-#endif
-constexpr int kOwnList = MI_OWN_LIST;            // list entries a class should have, at most
-constexpr int kOwnLog2S = MI_OWN_LOG2S;          // log2 of the workgroups that share a class
-#ifndef MI_OWN_TOKENS
-#define MI_OWN_TOKENS 8
-#endif
-constexpr int kOwnTokens = MI_OWN_TOKENS;        // tokens per workgroup, at least
-#ifndef MI_OWN_HEAVY
-#define MI_OWN_HEAVY 16
-#endif
-constexpr int kHeavy = MI_OWN_HEAVY;             // rows of a run that the whole workgroup adds
-// Vectors per thread per staged batch of a long run (32 KB of LDS with 16-byte vectors, 16 KB with scalars).
+// Neighbouring values, token backward in us, 64 or 768 columns of 50257 ids:
+//   kOwnLog2S 1 / 2 / 3    16384 tokens x 768, text 54.3 / 36.1 / 33.1, uniform 26.2 /
+//                          26.5 / 28.1; 16384 x 64 uniform 10.8 / 12.1 / 13.9
+//   kOwnTokens 4 / 8 / 16  1000 x 768 uniform 5.9 / 6.9 / 8.9, text 8.6 / 10.1 / 11.5;
+//                          2048 x 64 uniform 6.1 / 5.5 / 6.4, x 768 text 10.8 / 9.8 / 10.2
+//   kHeavy 8 / 16 / 32     2048 x 64 text 11.5 / 8.8 / 8.8; 512 x 768 of 65 ids, text 10.3 /
+//                          10.2 / 12.1, uniform 10.7 / 7.4 / 7.4
+constexpr int kOwnList = 256;                    // list entries a class should have, at most
+constexpr int kOwnLog2S = 2;                     // log2 of the workgroups that share a class
+constexpr int kOwnTokens = 8;                    // tokens per workgroup, at least
+constexpr int kHeavy = 16;                       // rows of a run that the class's workgroups share
+// Vectors per thread per staged batch of a long run (32 KB of LDS with 16-byte
+// vectors, 16 KB with scalars).
 template <int W>
 constexpr int heavy_vecs() {
     return W == 4 ? 4 : 8;
 }
-constexpr int kSlotBits = 11;                    // list slots fit: 2^11 = kOwnCap
+constexpr int kSlotBits = 11;                    // bits of a list slot in a key
+static_assert(kOwnCap == 1 << kSlotBits, "a list slot fits its bits");
+static_assert(kOwnCap % kHeavy == 0, "s_heavy holds every long run of a list");
 constexpr int kRankMax = 192;                    // longest list sorted by rank;
 constexpr int kRankWide = 384;                   // the same in place of two digits or more,
 constexpr int kRankTies = 128;                   // and with keys that do not hold the slot
@@ -245,12 +246,12 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
                      const int* __restrict__ ids, const float* __restrict__ g,
                      float* __restrict__ table, float* __restrict__ gpos) {
     constexpr int kSpan = kOwnThreads * PER;       // positions per pass
-    // Grad rows per group of loads in a short run: as many as the registers
-    // of NCH column vectors per lane leave room for.
     constexpr int kHeavyU = heavy_vecs<W>();
     constexpr unsigned kBins = kOwnThreads * kHeavyU * W / kOwnWaves;  // counts kept in s_stage
     constexpr int kBinBits = 31 - __builtin_clz(kBins);
     static_assert(kBins == 1u << kBinBits && kBins % kOwnThreads == 0, "digits of whole bits");
+    // Grad rows per group of loads in a short run: as many as the registers
+    // of NCH column vectors per lane leave room for.
     constexpr int kBatch = NCH == 1 ? 8 : NCH == 2 ? 4 : 2;
     // The list: keys and positions, [0] in position order, sorted in [srt]
     // (with room for the padding that the rank sort reads).  A key is the
@@ -971,12 +972,7 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
     // updates start as soon as the list is built (config-2 step 58.8 ->
     // 58.3 us against finishing the position sums first).
     if constexpr (POS) {
-        if (pv0 < pvec) {
-            if constexpr (PRE > 0)
-                pos_rest(pv0, PRE, s_pacc[threadIdx.x]);
-            else
-                pos_rest(pv0, 0, vload<W>(gpos, pv0));
-        }
+        if (pv0 < pvec) pos_rest(pv0, PRE, s_pacc[threadIdx.x]);
         pos_others();
     }
 }
