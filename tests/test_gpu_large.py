@@ -112,8 +112,7 @@ def _bwd_bound(ref):
     return BWD_ATOL * s + BWD_RTOL * ref.abs()
 
 
-def test_layernorm_past_2_31_elements(dev):
-    R, C = (1 << 21) + 37, 1024                       # 2,147,521,536 elements
+def _layernorm(dev, R, C):
     _need(56)
     note(f"large layernorm rows={R} cols={C}")
     gen = _gen(31)
@@ -141,7 +140,7 @@ def test_layernorm_past_2_31_elements(dev):
     g64, b64 = gamma.double(), beta.double()
     sg = torch.zeros(C, dtype=torch.float64, device=dev)
     sb, qg, qb = torch.zeros_like(sg), torch.zeros_like(sg), torch.zeros_like(sg)
-    for a, b in _chunks(R, 1 << 17):
+    for a, b in _chunks(R, (1 << 27) // C):
         x64, d64 = x[a:b].double(), dy[a:b].double()
         mu = x64.mean(1, keepdim=True)
         xc = x64 - mu
@@ -164,6 +163,38 @@ def test_layernorm_past_2_31_elements(dev):
     ref_g, ref_b = sg + 0.5, sb - 0.25
     _close("dgamma", dg, ref_g, COL_RTOL * (ref_g.abs() + qg.sqrt()), 0)
     _close("dbeta", db, ref_b, COL_RTOL * (ref_b.abs() + qb.sqrt()), 0)
+
+
+def test_layernorm_past_2_31_elements(dev):
+    _layernorm(dev, (1 << 21) + 37, 1024)             # 2,147,521,536 elements
+
+
+def test_narrow_layernorm_past_2_31_elements(dev):
+    _layernorm(dev, E31 // 96 + 37, 96)               # two rows a wave
+
+
+# Row lanes, rows of whole vectors and ragged ones with a last element past
+# the last vector.  Integer gradients: the column sums are exact in any order.
+@pytest.mark.parametrize("C", [96, 333])
+def test_narrow_column_sums_past_2_31_elements(dev, C):
+    R = E31 // C + 41
+    _need(40)
+    note(f"large column sums rows={R} cols={C}")
+    gen = _gen(C)
+    x = torch.randn(R, C, device=dev, generator=gen)
+    g = torch.empty(R, C, device=dev).random_(-4, 5, generator=gen)
+    gin, db, dall = _nan(R, C), torch.full((C,), 3.0, device=dev), torch.full((C,), -5.0, device=dev)
+    M.relu_backward_with_bias_backward(x, g, gin, db, R, C)
+    M.bias_backward(g, dall, R, C)
+    torch.cuda.synchronize()
+    sums = torch.zeros(2, C, dtype=torch.float64, device=dev)
+    for a, b in _chunks(R, (1 << 27) // C):
+        ref = torch.where(x[a:b] > 0, g[a:b], torch.zeros_like(g[a:b]))
+        _same("grad_in", gin[a:b], ref, a)
+        sums[0] += ref.sum(0, dtype=torch.float64)
+        sums[1] += g[a:b].sum(0, dtype=torch.float64)
+    _same("relu dbias", db, (sums[0] + 3.0).float(), 0)
+    _same("dbias", dall, (sums[1] - 5.0).float(), 0)
 
 
 def _gelu64(u):

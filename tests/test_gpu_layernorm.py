@@ -240,3 +240,30 @@ def test_wide_sweep_config4(dev):
 def test_layernorm_width_edges(dev, rows, cols):
     test_layernorm_forward_backward(dev, rows, cols, rows + cols)
     test_residual_layernorm_and_backward_residual(dev, rows, cols, rows + cols)
+
+
+# Rows with a NaN, an infinity or the lowest float among rows that share their
+# wave or workgroup: those others keep their bits, forward and backward, and
+# the affected rows and the column sums that they reach are not finite.
+@pytest.mark.parametrize("rows,cols", [(70, 60), (70, 96), (2100, 128), (30, 516), (9, 1026), (7, 5120)])
+def test_non_finite_rows_stay_alone(dev, rows, cols):
+    x, gamma, beta, g = ln_inputs(rows, cols, rows + cols)
+    bad = {1: np.nan, 4: np.inf, rows - 1: np.finfo(np.float32).min}
+    xb = x.copy()
+    for r, v in bad.items():
+        xb[r, r % cols] = v
+    out = []
+    for a in (x, xb):
+        X, G, Gm = dev_t(a), dev_t(g), dev_t(gamma)
+        y, dx = torch.empty(rows, cols, device=dev), torch.empty(rows, cols, device=dev)
+        mean, rstd = torch.empty(rows, device=dev), torch.empty(rows, device=dev)
+        dg, db = torch.zeros(cols, device=dev), torch.zeros(cols, device=dev)
+        M.layernorm_forward_save(X, Gm, dev_t(beta), y, mean, rstd, rows, cols, 1e-5)
+        M.layernorm_backward(G, X, mean, rstd, Gm, dx, dg, db, rows, cols)
+        out.append([host(t) for t in (y, mean, rstd, dx, dg, db)])
+    keep = np.array([r not in bad for r in range(rows)])
+    for name, want, got in zip(("y", "mean", "rstd", "dx"), out[0], out[1]):
+        assert_exact(name, got[keep], want[keep])
+    assert not np.isfinite(out[1][0][[1, 4]]).any() and not np.isfinite(out[1][3][[1, 4]]).any()
+    assert np.isnan(out[1][4]).all()            # dgamma: NaN normalised values reach every column
+    assert_exact("dbeta", out[1][5], out[0][5])  # sums of grad_out alone

@@ -219,3 +219,36 @@ def test_softmax_time_against_the_scalar_accesses(dev, rows, cols):
     # 0.99 measured; 1.18 and 1.08 with 16-byte accesses at every width and the
     # streaming hint on the loads of every row past 4096 columns
     assert t[0] <= 1.06 * t[1]
+
+
+# Masked logits (-inf, the lowest float) next to ordinary ones, and rows with a
+# NaN or +inf, in every row shape with 16-byte accesses and off 16 bytes.
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("cols", [64, 100, 1028, 2052, 4100, 8196, 32000, 65536])
+def test_masked_and_non_finite_logits(dev, cols, off):
+    rows = 9
+    x, t = _logits(rows, cols, cols)
+    lowest = np.finfo(np.float32).min
+    x[1, 1::2] = -np.inf
+    x[2, ::3] = lowest
+    x[3, :-1] = lowest                  # one logit left
+    x[5, cols // 2] = np.nan
+    x[7, cols - 1] = np.inf
+    t[1], t[2], t[3] = 0, 1, cols - 1
+    buf = torch.empty(rows * cols + 1, device="cuda")
+    X, Y = buf[off:off + rows * cols], torch.empty(rows * cols + 1, device="cuda")[off:off + rows * cols]
+    X.copy_(dev_t(x).reshape(-1))
+    M.softmax_forward(X, Y, rows, cols)
+    y = host(Y).reshape(rows, cols)
+    fine = [0, 1, 2, 3, 4, 6, 8]
+    assert_fwd("softmax", y[fine], O.softmax_forward_f64(x[fine]))
+    assert (y[1, 1::2] == 0).all() and (y[2, ::3] == 0).all() and y[3, -1] == 1
+    assert np.isnan(y[[5, 7]]).all()
+    losses, lout = torch.empty(rows, device="cuda"), torch.empty(1, device="cuda")
+    M.cross_entropy_forward_v2(X, dev_t(t), Y, losses, lout, rows, cols)
+    l64, g64 = O.cross_entropy_f64(x[fine], t[fine])
+    assert_bwd("gradient", host(Y).reshape(rows, cols)[fine] * np.float32(rows), g64)
+    lg = host(losses)
+    pt = np.exp(-l64)
+    assert (np.abs(lg[fine] - l64) <= 1e-6 + 1e-5 * np.abs(l64) + 1.01e-9 / pt).all()
+    assert np.isnan(lg[[5, 7]]).all()
