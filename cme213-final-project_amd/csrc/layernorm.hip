@@ -1017,15 +1017,17 @@ BwdPlan plan_bwd(int rows, int cols, bool vec4, bool add) {
     // 81 us against 69; the residual form gains at 771 columns, [16384, 771]
     // 42.6 against 47.8 us, and at 1001 only where the tensors are in the
     // last-level cache: [16384, 1001] 41.8 against 43.1, from memory 56.0
-    // against 52.4).  Wider rows use the block-per-row kernel.
+    // against 52.4).  N = 5 serves 1025 to 1280 columns (with 6, a sixth of the
+    // loads was of clamped columns: [4096, 1026] 15.8 -> 14.8 us, [16384, 1026] 43.3 ->
+    // 38.9).  Wider rows use the block-per-row kernel.
     static const int kG[] = {1, 4, 8};
-    static const int kN[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    static const int kN[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
     const int max_n = p.W == 4 ? 6 : 16;
     for (int gi = 0; gi < 3 && !p.N; ++gi) {
         const int g = kG[gi];
         const int need = (nv + g * kWave - 1) / (g * kWave);
         for (int n : kN)
-            if (n >= need && n <= max_n) {
+            if (n >= need && n <= max_n && (n != 5 || p.W == 1)) {
                 p.N = n;
                 p.G = g;
                 break;
@@ -1099,6 +1101,7 @@ void dispatch_bwd_n(const BwdPlan& p, hipStream_t st, const float* g, const floa
     }
     if constexpr (W == 1) {
         switch (p.N) {
+            case 5: launch_bwd_group<W, 5, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
             case 8: launch_bwd_group<W, 8, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
             case 12: launch_bwd_group<W, 12, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;
             case 16: launch_bwd_group<W, 16, G, ADD>(p, st, g, x, m, s, gamma, gx, part, rows, cols); break;

@@ -236,6 +236,7 @@ def test_wide_sweep_config4(dev):
     (65, 132), (19, 1025), (7, 1281), (300, 1538), (5, 4095), (4, 4097), (3, 8191), (2, 8195),
     (1024, 260), (1025, 260), (2, 1024), (1024, 516), (33, 257), (16, 1600), (1000, 70),
     (3, 12289), (6, 4100), (300, 5120), (3, 12292), (2, 16388), (2, 49156), (700, 640 + 255),
+    (9, 1279), (259, 1280), (260, 1281),
 ])
 def test_layernorm_width_edges(dev, rows, cols):
     test_layernorm_forward_backward(dev, rows, cols, rows + cols)
