@@ -317,16 +317,16 @@ __global__ __launch_bounds__(1024) void rowband_kernel(const void* w0, const voi
 // rows (one or two waves per CU at 256 or 512 columns) and falls back to
 // 4-byte accesses where rows do not start on 16 bytes.  Memory-bound; half
 // ReLU forward + backward [4096, 1024] 21.8 -> 16.9 us, [16384, 333] 35.8 ->
-// 22.4 us.  Here a workgroup takes RL consecutive
-// rows at a time as one contiguous run of sv = RL * cols / 4 vectors, RL a
-// multiple of 4 / gcd(cols, 4), so that every run starts on 16 bytes: thread
-// t owns the super-columns of vectors t + k * T, keeps their biases and sums
-// in registers, and a vector may span two rows.  At the end the RL sums of
-// each column are added through LDS, as eight interleaved sums and then
-// pairwise (in sequence they were up to 256 terms: [65536, 16] column sums,
-// relative 2-norm against float64, 3.7e-7, 1.5e-7 so), and the workgroup writes
-// one partial row, as a band does.  The at most 3 elements past the
-// last whole vector are the last row's: workgroup 0 takes them one by one.
+// 22.4 us.  Here a workgroup takes RL consecutive rows at a time as one
+// contiguous run of sv = RL * cols / 4 vectors, RL a multiple of 4 / gcd(cols,
+// 4), so that every run starts on 16 bytes: thread t owns the super-columns of
+// vectors t + k * T, keeps their biases and sums in registers, and a vector may
+// span two rows.  At the end the RL sums of each column are added through LDS:
+// eight interleaved sums over whole groups of eight rows, added pairwise, then
+// the last rows (all in sequence they were up to 256 terms: [65536, 16] column
+// sums, relative 2-norm against float64, 3.7e-7, 1.5e-7 so).  The workgroup then
+// writes one partial row, as a band does.  The at most 3 elements past the last
+// whole vector are the last row's: workgroup 0 takes them one by one.
 // ---------------------------------------------------------------------------
 template <int NC, class Op, class Op1>
 __global__ __launch_bounds__(1024) void rowlane_kernel(const void* w0, const void* w1,
@@ -398,16 +398,15 @@ __global__ __launch_bounds__(1024) void rowlane_kernel(const void* w0, const voi
         float s[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) s[i] = 0.0f;
-        for (int x0 = c; x0 < n; x0 += 8 * cols)
+        int x = c;
+        for (; x + 7 * cols < n; x += 8 * cols)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int x = x0 + i * cols;
-                s[i] += x < n ? lane_sums[x] : 0.0f;
-            }
+            for (int i = 0; i < 8; ++i) s[i] += lane_sums[x + i * cols];
 #pragma unroll
         for (int h = 4; h >= 1; h /= 2)
 #pragma unroll
             for (int i = 0; i < h; ++i) s[i] += s[i + h];
+        for (; x < n; x += cols) s[0] += lane_sums[x];
         if (blockIdx.x == 0 && c >= cols - tail) s[0] += lane_sums[n + c - (cols - tail)];
         prow[c] = s[0];
     }
