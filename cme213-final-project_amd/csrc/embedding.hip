@@ -189,12 +189,13 @@ __global__ __launch_bounds__(256) void pos_bwd_kernel(const float* __restrict__ 
 // bit-identical whichever workgroup or wave adds it.
 //
 // What bounds it depends on the ids.  Uniform over a large vocabulary (16384
-// tokens, D = 768, V = 50257: fwd + bwd 53.3 us, 54.6 with one workgroup per
-// class and every run on one wave): the random 3 KB rows, after ~9 us of
-// scan and sort in which only the position rows stream.  Frequencies of text
-// on the same shape: the longest runs, 66 us against 208 us when one wave
-// added each (a memory round trip per two rows of a 466-row run).  A few
-// characters (32 x 256 tokens of 65 ids, D = 512): 23 us against 287 us.
+// tokens, D = 768, V = 50257: fwd + bwd 53.4 us, 54.2 with one workgroup per
+// class and every run on one wave): the random 3 KB rows, behind the scan and
+// the sort, during which only the position rows stream (the token backward
+// takes 26.5 us, and 12.1 with rows of 64 columns).  Frequencies of text on the
+// same shape: the longest runs, 67 us against 202 us when one wave added each
+// (a memory round trip per two rows of a 466-row run).  A few characters (32 x
+// 256 tokens of 65 ids, D = 512): 23 us against 287 us.
 // ---------------------------------------------------------------------------
 constexpr int kOwnWaves = 8;
 constexpr int kOwnThreads = kOwnWaves * kWave;   // 512

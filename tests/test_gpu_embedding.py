@@ -62,8 +62,8 @@ def test_reference_embedding_test_case(dev):
     (50257, 64, 33, 1000, 50257),
     (300, 32, 1, 16385, 300),        # one token into the second pass, long runs
     (70000, 16, 2, 9000, 0),         # trusted ids, 18000 tokens
-    (2000, 1600, 2, 500, 2000),      # GPT-2-XL width: 4 vectors per lane, 2 column chunks
-    (500, 1030, 1, 700, 500),        # scalar columns, 5 column chunks
+    (2000, 1600, 2, 500, 2000),      # GPT-2-XL width: 3 vectors per lane, 3 column chunks
+    (500, 1030, 1, 700, 500),        # scalar columns, 6 column chunks
 ])
 def test_embedding_forward_backward(dev, V, D, B, T, vocab_arg):
     note(f"embedding V={V} D={D} B={B} T={T} vocab_arg={vocab_arg}")
@@ -247,7 +247,7 @@ def _runs(lengths, vocab, n, seed):
     (5000, 36, 16384, (2040, 1500, 600, 40), 5000),         # a list near its capacity
     (65, 512, 8192, (900, 800, 17), 65),                    # few ids: many slices per class
     (65, 40, 16385, (5000, 300), 65),                       # empty last slices, list overflow
-    (3, 1030, 700, (300, 20), 3),                           # scalar columns, 5 column chunks
+    (3, 1030, 700, (300, 20), 3),                           # scalar columns, 6 column chunks
     (70000, 16, 9000, (200, 150, 16), 0),                   # trusted ids
     (60000, 32, 60000, (3000, 2100, 500, 16), 60000),       # several scans into one list
     # lists of more and of fewer than 128 entries in classes of more ids than
