@@ -9,7 +9,7 @@ the block-per-row fallbacks, vector (W = 4) against scalar columns (width not
 a multiple of 4, or a tensor that starts 4 bytes into its allocation), the
 flat against the row-band form of the bias operators (one to four column
 vectors per row-band thread), and the embedding
-backward's owner count (a power of two from about 32 tokens each)."""
+backward's workgroup count (a power of two, of at least 8 tokens each)."""
 import numpy as np
 import pytest
 import torch
