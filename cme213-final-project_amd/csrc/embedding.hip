@@ -224,9 +224,8 @@ constexpr int heavy_vecs() {
 constexpr int kSlotBits = 11;                    // bits of a list slot in a key
 static_assert(kOwnCap == 1 << kSlotBits, "a list slot fits its bits");
 static_assert(kOwnCap % kHeavy == 0, "s_heavy holds every long run of a list");
-constexpr int kRankMax = 192;                    // longest list sorted by rank;
-constexpr int kRankWide = 384;                   // the same in place of two digits or more,
-constexpr int kRankTies = 128;                   // and with keys that do not hold the slot
+constexpr int kRankMax = 128;                    // longest list sorted by rank, and
+constexpr int kRankWide = 384;                   // the same in place of two digits or more
 
 // Position gradient fused into the owner kernel (POS): the workgroups also
 // share out the seq * nv position column vectors, one per thread per round;
@@ -569,14 +568,16 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
 
     // Sorts list entries [0, L) by id, stably: short lists by rank, four
     // threads an entry, longer ones by counting, digit by digit of kBinBits
-    // bits, low digit first; one digit holds a class of up to kBins ids.  A
-    // digit costs about 2.3 us however long the list is, ranks grow with its
-    // square (11 us at 450), hence the lines (16384 uniform ids, 64 columns,
-    // lists of 128 on average, ranks up to 128 / up to 192: vocabulary 50257
-    // 13.0 / 12.2 us; 151936, two digits, 15.9 / 12.8; 24576 of 151936, lists of
-    // 192, ranks up to 192 / 256: 22.0 / 19.6).  One bit a pass, which calls
-    // without a vocabulary bound took for every list, cost 1 us a bit (16384 ids
-    // of 50257, no bound: 16.9 us, 12.8 now; 16 ids: 10.8, 4.7 now).
+    // bits, low digit first; one digit holds a class of up to kBins ids.  Ranks
+    // grow with the square of the list (11 us at 450 entries), a digit costs 1
+    // to 2 us however long it is, hence the lines (64 columns, us, ranks up to
+    // 64 / 128 / 192: 8192 uniform ids of 50257, lists of 64 on average, 11.4 /
+    // 10.2 / 10.2; 16384 of 50257, lists of 128, 12.4 / 12.5 / 12.1, of 5000 11.0 /
+    // 11.0 / 11.1; 2048 with the frequencies of 65 letters 8.3 / 8.2 / 9.3; two
+    // digits: 24576 of 151936, ranks up to 192 / 256 22.0 / 19.6).  One bit a
+    // pass, which calls without a vocabulary bound took for every list, cost 1
+    // us a bit (16384 ids of 50257, no bound: 16.9 us, 12.7 now; 16 ids: 10.8, 4.7
+    // now).
     //
     // Runs of at least kHeavy rows are added by the class's workgroups
     // together, by column slices; of the shorter runs a workgroup takes those
@@ -588,9 +589,9 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
         // No number of the list is above `top`.  Where the vocabulary bound
         // says little, the list does, and where the keys have no slot for
         // want of a bound they get one now.
-        unsigned top = qlim - 1u;
-        if (!slots || (top >= kBins && L > kRankWide)) {
-            if (!slots) kshift = 0;
+        unsigned top = L > 1 ? qlim - 1u : 0u;
+        if (!slots) kshift = 0;
+        if (L > 1 && (!slots || (top >= kBins && L > kRankWide))) {
             unsigned any = 0;
             for (int i = static_cast<int>(threadIdx.x); i < L; i += kOwnThreads) any |= s_key[i];
             any = wave_or(any);
@@ -606,7 +607,9 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
                 kshift = kSlotBits;
             }
         }
-        if (L <= (kshift == 0 ? kRankTies : top < kBins ? kRankMax : kRankWide)) {
+        if (top == 0) {
+            srt = 0;  // one id at most: sorted as it is
+        } else if (L <= (top < kBins || kshift == 0 ? kRankMax : kRankWide)) {
             srt = 1;
             if (threadIdx.x < 16) s_key[L + threadIdx.x] = 0xffffffffu;
             __syncthreads();
@@ -650,13 +653,23 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
             const int span = (L + kOwnThreads - 1) / kOwnThreads * kWave;
             int* const cnt = reinterpret_cast<int*>(s_stage);  // [wave][kBins]
             int lo = kshift;
-            const int hi = kshift + 32 - __builtin_clz(top | 1u);
+            const int hi = kshift + 32 - __builtin_clz(top);
             srt = 0;
 #pragma unroll 1
             for (; lo < hi; lo += kBinBits) {
                 const int nbits = hi - lo < kBinBits ? hi - lo : kBinBits;
-                for (unsigned i = threadIdx.x; i < kOwnWaves * kBins; i += kOwnThreads)
-                    cnt[i] = 0;
+                // Thread t takes the digits t * kPer + [0, kPer) of those there
+                // are (no number has a bit from hi up); waves past them have
+                // nothing to clear or add.
+                constexpr int kPer = kBins / kOwnThreads;
+                int* const mine = cnt + static_cast<int>(threadIdx.x) * kPer;
+                const bool some = threadIdx.x * kPer < (1u << nbits);
+                if (some) {
+#pragma unroll
+                    for (int b = 0; b < kPer; ++b)
+#pragma unroll
+                        for (int w = 0; w < kOwnWaves; ++w) mine[w * kBins + b] = 0;
+                }
                 __syncthreads();
                 auto digit = [&](unsigned key) __attribute__((always_inline)) {
                     return (key >> lo) & (kBins - 1u);
@@ -687,14 +700,13 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
                     wave_order();
                 }
                 __syncthreads();
-                // Thread t takes the digits t * kPer + [0, kPer).
-                constexpr int kPer = kBins / kOwnThreads;
                 int bsum = 0;
+                if (some) {
 #pragma unroll
-                for (int b = 0; b < kPer; ++b)
+                    for (int b = 0; b < kPer; ++b)
 #pragma unroll
-                    for (int w = 0; w < kOwnWaves; ++w)
-                        bsum += cnt[w * kBins + static_cast<int>(threadIdx.x) * kPer + b];
+                        for (int w = 0; w < kOwnWaves; ++w) bsum += mine[w * kBins + b];
+                }
                 int upto = bsum;  // inclusive sum over the wave's lanes
 #pragma unroll
                 for (int o = 1; o < kWave; o *= 2) {
@@ -706,15 +718,16 @@ emb_bwd_owner_kernel(int n, int vocab, int dim, int batch, int seq, int cfg,
                 int run = upto - bsum;
 #pragma unroll
                 for (int w = 0; w < kOwnWaves; ++w) run += w < wave ? s_wsum[w] : 0;
+                if (some) {
 #pragma unroll
-                for (int b = 0; b < kPer; ++b)
+                    for (int b = 0; b < kPer; ++b)
 #pragma unroll
-                    for (int w = 0; w < kOwnWaves; ++w) {
-                        int* const c = &cnt[w * kBins + static_cast<int>(threadIdx.x) * kPer + b];
-                        const int v = *c;
-                        *c = run;
-                        run += v;
-                    }
+                        for (int w = 0; w < kOwnWaves; ++w) {
+                            const int v = mine[w * kBins + b];
+                            mine[w * kBins + b] = run;
+                            run += v;
+                        }
+                }
                 __syncthreads();
 #pragma unroll
                 for (int q = 0; q < kQ; ++q) {
