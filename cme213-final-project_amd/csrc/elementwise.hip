@@ -873,28 +873,37 @@ struct LanePlan {
 };
 
 // Rows take as many row lanes as fill 1024 threads while the runs still go
-// round kLaneBlocks workgroups, up to 2048 columns, and up to kLaneRagged where
-// the width is no multiple of 4.  Wider rows stay with the row bands: GELU
-// backward + dbias by row lanes / by bands [4096, 2048] 20.8 / 21.8 us, [16384,
-// 2048] 68.6 / 72.1, [8192, 1024] 20.6 / 31.0, but [512, 2560] 8.1 / 7.7, [8192,
-// 3072] 52.2 / 51.5, [4096, 8192] 79.2 / 76.9.  Ragged widths, lanes over bands in
-// time, tensors in the last-level cache / in HBM: [8192, 999] 0.99 / 0.70, [8192,
-// 1101] 0.98 / 0.71, [8192, 1201] 1.05 / 0.76, [8192, 1538] 1.09 / 0.85, [4096, 1701]
-// 1.19 / 0.98, [4096, 2302] 1.15 / 0.99, [1000, 4094] 1.32 / 1.10, [256, 8190] 1.78 /
-// 1.65: a run of one row unit leaves a CU one workgroup with one to four
-// vectors a thread in flight (two runs in flight: 1.0 to 1.1 times slower).
+// round kLaneBlocks workgroups, up to 2048 columns.  Wider rows stay with the row
+// bands: GELU backward + dbias by row lanes / by bands [4096, 2048] 20.8 / 21.8 us,
+// [16384, 2048] 68.6 / 72.1, [8192, 1024] 20.6 / 31.0, but [512, 2560] 8.1 / 7.7, [8192,
+// 3072] 52.2 / 51.5, [4096, 8192] 79.2 / 76.9.  Widths that are no multiple of 4 do
+// so up to kLaneRagged columns, and with kLaneRaggedRows rows or more up to
+// `ragged`: kRaggedWord columns where a 4-byte tensor is read beside the gradient
+// and kRaggedMost otherwise.  Time by lanes over time by bands, GELU / 16-bit mask
+// / column sums, tensors from memory and (in brackets) in the last-level cache:
+// [8192, 999] 0.70 (0.98) / 0.62 (0.87) / 0.70 (0.71), [8192, 1201] 0.75 (1.04) / 0.65
+// (0.94) / 0.76 (0.72), [8192, 1538] 0.84 (1.10) / 0.73 (0.99) / 0.99 (0.97), [8192, 1701]
+// 0.98 (1.22) / 0.81 (1.08) / 0.67 (0.77), [4096, 1802] 0.94 (1.09) / 0.81 (1.00) / 1.08
+// (1.04), [4096, 2302] 1.00 (1.14) / 0.88 (1.03) / 1.00 (1.07), [256, 8190] 1.62 (1.95) /
+// 1.33 (1.45) / 1.38 (1.23); few rows [1000, 1026] 1.00 (1.03) / 0.92 (1.02) / 0.85
+// (1.01), [1000, 1538] 1.04 (1.06) / 1.02 (0.99) / 0.89 (1.00): a run of one row unit
+// leaves a CU one workgroup with one to four vectors a thread in flight (two runs
+// in flight: 1.0 to 1.1 times slower).
 // Below 16 columns the plain bands stay (a run must hold the tail elements'
 // columns, and such rows are never large).
 constexpr int kLaneBlocks = 256;
 constexpr int kLaneThreads = 1024;
 constexpr int kLaneRagged = 1152;
-constexpr int kLaneNC = 2;  // vectors per thread: 4 rows of kLaneRagged columns at most
-static_assert(kLaneRagged <= kLaneNC * 1024, "the widest run fits the threads");
+constexpr int kLaneRaggedRows = 2048;
+constexpr int kRaggedMost = 2048, kRaggedWord = 1600;
+constexpr int kLaneNC = 2;  // vectors per thread: 4 rows of kRaggedMost columns at most
+static_assert(kRaggedMost <= kLaneNC * 1024, "the widest run fits the threads");
 
-LanePlan plan_lanes(int rows, int cols) {
+LanePlan plan_lanes(int rows, int cols, int ragged) {
     LanePlan p;
     const int unit = cols % 4 == 0 ? 1 : cols % 2 == 0 ? 2 : 4;  // rows of a 16-byte aligned run
-    if (cols < 16 || cols > (unit == 1 ? 2048 : kLaneRagged)) return p;
+    const int most_cols = unit == 1 ? 2048 : rows < kLaneRaggedRows ? kLaneRagged : ragged;
+    if (cols < 16 || cols > most_cols) return p;
     const int sv1 = unit * cols / 4;
     int m = kLaneThreads / sv1;  // units per run
     const int most = rows / (unit * kLaneBlocks);
@@ -963,12 +972,12 @@ int launch_rowtile_reduce(const char* name, Op op, const float* bias, float* dbi
 
 // A reducing operator as its 16-byte form `op` and scalar form `op1` (the
 // same pointers); `aligned`: the tensors' own alignment allows 16-byte
-// accesses at every fourth element.
+// accesses at every fourth element; `ragged`: see plan_lanes.
 template <class Op, class Op1>
 int launch_reduce(const char* name, Op op, Op1 op1, bool aligned, const float* bias, float* dbias,
-                  int rows, int cols, hipStream_t st) {
+                  int rows, int cols, hipStream_t st, int ragged) {
     if (aligned) {
-        const LanePlan p = plan_lanes(rows, cols);
+        const LanePlan p = plan_lanes(rows, cols, ragged);
         if (p.rl > 0)
             return launch_rowlane_reduce<Op, Op1>(name, p, op, bias, dbias, rows, cols, st);
         // 16-byte loads of the bias need its alignment too
@@ -995,7 +1004,7 @@ size_t mi_bias_backward_workspace(int rows, int cols) {
     if (rows <= 0 || cols <= 0) return 0;
     // the band plans of 16-byte and 4-byte accesses and the row-lane plan can
     // differ; report the largest
-    int parts = plan_lanes(rows, cols).blocks;
+    int parts = plan_lanes(rows, cols, kRaggedMost).blocks;
     for (int nv : {cols / 4, cols}) {
         const int p = plan_reduce_parts(rows, nv);
         if (p > parts) parts = p;
@@ -1087,7 +1096,7 @@ int mi_bias_backward(const float* grad, float* dbias, int rows, int cols, void* 
     if (rows == 0) return MI_OK;
     if (!grad || !dbias) return set_error(MI_ERR_INVALID_ARG, "%s: NULL", name);
     return launch_reduce(name, ColSumOp<4>{grad}, ColSumOp<1>{grad}, all_aligned({grad}), nullptr,
-                         dbias, rows, cols, to_stream(stream));
+                         dbias, rows, cols, to_stream(stream), kRaggedMost);
 }
 
 int mi_relu_backward_with_bias_backward(const float* mask, const float* grad_out, float* grad_in,
@@ -1100,7 +1109,7 @@ int mi_relu_backward_with_bias_backward(const float* mask, const float* grad_out
     return launch_reduce(name, ReluBwdBiasOp<4>{mask, grad_out, grad_in},
                          ReluBwdBiasOp<1>{mask, grad_out, grad_in},
                          all_aligned({mask, grad_out, grad_in}), nullptr, dbias, rows, cols,
-                         to_stream(stream));
+                         to_stream(stream), kRaggedWord);
 }
 
 int mi_gelu_backward_with_bias_backward(const float* in, const float* bias,
@@ -1114,7 +1123,7 @@ int mi_gelu_backward_with_bias_backward(const float* in, const float* bias,
     return launch_reduce(name, GeluBwdBiasOp<4>{in, grad_out, grad_in},
                          GeluBwdBiasOp<1>{in, grad_out, grad_in},
                          all_aligned({in, grad_out, grad_in}), bias, dbias, rows, cols,
-                         to_stream(stream));
+                         to_stream(stream), kRaggedWord);
 }
 
 }  // extern "C"
@@ -1179,7 +1188,7 @@ int relu_bwd_mask16(const char* name, const void* mask, const float* grad_out, f
     return launch_reduce(name, ReluBwdMask16Op<4, T>{m, grad_out, grad_in},
                          ReluBwdMask16Op<1, T>{m, grad_out, grad_in},
                          aligned8(m) && all_aligned({grad_out, grad_in}), nullptr, dbias, rows,
-                         cols, to_stream(stream));
+                         cols, to_stream(stream), kRaggedMost);
 }
 
 }  // namespace

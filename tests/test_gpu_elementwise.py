@@ -205,13 +205,16 @@ def _offset(a, offset):
 
 
 # Row lanes: widths around their bounds (16 columns, 512 whole vectors, 1152
-# columns of 2- and 4-row runs), row counts that leave a partial run, one to
-# three elements past the last vector, and tensors off 16 bytes.
+# columns of 2- and 4-row runs, and 1600 and 2048 with 2048 rows), row counts that
+# leave a partial run, one to three elements past the last vector, and tensors
+# off 16 bytes.
 @pytest.mark.parametrize("rows,cols,off", [
     (1, 15, 0), (1, 16, 0), (1, 17, 0), (3, 18, 0), (2, 19, 0), (255, 64, 0), (2049, 30, 0),
     (1025, 511, 0), (1027, 512, 0), (2050, 127, 0), (513, 2048, 0), (513, 2052, 0), (300, 1025, 0),
     (77, 2047, 0), (601, 4094, 0), (5, 4095, 0), (6, 4097, 0), (9, 8190, 0), (259, 8194, 0),
     (1030, 96, 1), (7, 1002, 3), (2049, 1151, 0), (515, 1150, 0), (3, 1153, 0), (300, 1154, 0),
+    (2048, 1599, 0), (2047, 1598, 0), (2048, 1602, 0), (2049, 2046, 0), (2048, 2047, 0),
+    (2048, 2049, 0),
 ])
 def test_column_sums_row_lanes(dev, rows, cols, off):
     note(f"row lanes rows={rows} cols={cols} off={off}")
@@ -261,7 +264,7 @@ def test_gelu_backward_ragged_widths_time(dev, rows, cols):
     t = batch_us(*(M.bind("mi_gelu_backward_with_bias_backward", x[o:o + n], bias, g[o:o + n],
                           gin[o:o + n], db, rows, cols) for o in (0, 1)))
     note(f"gelu backward [{rows}, {cols}]: {t[0]:.2f} us, {t[1]:.2f} us off 16 bytes")
-    # at most 1.0 measured; 1.2 to 1.8 with row lanes at every ragged width
+    # at most 1.0 measured; 1.1 to 2.0 with row lanes at every ragged width
     assert t[0] <= 1.15 * t[1]
 
 
