@@ -192,7 +192,7 @@ __global__ __launch_bounds__(256) void pos_bwd_kernel(const float* __restrict__ 
 // tokens, D = 768, V = 50257: fwd + bwd 53.4 us, 54.2 with one workgroup per
 // class and every run on one wave): the random 3 KB rows, behind the scan and
 // the sort, during which only the position rows stream (the token backward
-// takes 26.5 us, and 12.1 with rows of 64 columns).  Frequencies of text on the
+// takes 26.9 us, and 12.6 with rows of 64 columns).  Frequencies of text on the
 // same shape: the longest runs, 67 us against 202 us when one wave added each
 // (a memory round trip per two rows of a 466-row run).  A few characters (32 x
 // 256 tokens of 65 ids, D = 512): 23 us against 287 us.
